@@ -87,3 +87,27 @@ def test_gather_and_scatter_add_rows(backend):
     for i in range(n):
         want[idx[i]] = want[idx[i]] + (np.float32(w[i]) * part[i]).astype(np.float32)
     assert np.array_equal(host_f32(dst).view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 4), (2, 513), (64, 512), (65, 516), (256, 1), (257, 1280), (1000, 77),
+                                       (1281, 132)])
+@pytest.mark.parametrize("pick", ["distinct", "repeats", "one"])
+def test_scatter_add_rows_in_order(backend, rows, cols, pick):
+    """Bitwise the rows added one by one: distinct indices (an expert's rows),
+    indices repeated across the scan's steps, and every row onto one."""
+    g = np.random.default_rng(rows * cols)
+    count = rows + 3
+    idx = {"distinct": g.permutation(count)[:rows], "repeats": g.integers(0, max(1, rows // 3), rows),
+           "one": np.full(rows, 2)}[pick].astype(np.int64)
+    dst0, w, part = normal(530, (count, cols)), normal(531, rows), normal(532, (rows, cols))
+    # one element past the start: a base that allows no 16-byte access
+    for shift in (0, 1):
+        buf = torch.zeros(count * cols + 4, device="cuda")
+        dst = buf[shift:shift + count * cols].view(count, cols)
+        dst.copy_(dev_f32(dst0))
+        backend.scatter_add_rows(dst, dev_i64(idx), dev_f32(w), dev_f32(part))
+        want = dst0.copy()
+        for i in range(rows):
+            want[idx[i]] = want[idx[i]] + (np.float32(w[i]) * part[i]).astype(np.float32)
+        assert np.array_equal(host_f32(dst).view(np.uint32), want.view(np.uint32)), f"shift {shift}"
+        assert torch.count_nonzero(buf[:shift]) == 0 and torch.count_nonzero(buf[shift + count * cols:]) == 0
