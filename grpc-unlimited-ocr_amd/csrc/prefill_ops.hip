@@ -5,11 +5,16 @@
 //
 // gemm_nt / gemm_nn: c[b] = alpha a[b] . b[b]^T (b rows k-contiguous) or
 // a[b] . b[b] (b rows n-contiguous), batched over slices `stride_*` elements
-// apart, leading dimensions given. A workgroup of 256 threads computes a
-// 64 x 64 tile of one slice; each thread a 4 x 4 block. k advances 16 at a
-// time through LDS, both operands held k-major there so that a thread reads
-// its 4 a values and 4 b values as two 16-byte loads per k. Sums are fp32
-// (fused multiply-adds), alpha applied to the finished sum. Any m, n, k.
+// apart, leading dimensions given, on the fp32 matrix cores
+// (v_mfma_f32_32x32x2f32: fp32 products and sums, two columns of k each, lane
+// half h supplying column 2 i + h of product i). No LDS for the operands: a
+// lane reads 16 consecutive bytes of its k-contiguous row (half h columns
+// 8 j + 4 h ..) and two half swaps put them in the products' order; the
+// n-contiguous operand is read as 32 consecutive floats per half. The next
+// span of k is in flight in registers while the current one multiplies.
+// Sums run over k in order, one fused multiply-add a column (past kGemmChain
+// columns: four such runs added in order), alpha applied to the finished
+// sum. Any m, n, k.
 //
 // gather_rows: dst[i] = src[index[i]]; scatter_add_rows: dst[index[i]] +=
 // weight[i] * src[i] for i in order (each column walks the rows in order, so
@@ -20,8 +25,10 @@
 namespace uocr_rocm {
 namespace {
 
-constexpr int kGM = 64, kGN = 64, kGK = 16;
-constexpr int kGemmBlock = 256;
+constexpr int kGemmTile = 32;  // rows and columns of one matrix-core product
+constexpr int kGemmWaves = 4;
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 struct GemmArgs {
   const float* a;
@@ -31,72 +38,189 @@ struct GemmArgs {
   int64_t lda, ldb, ldc;
   int64_t sa, sb, sc;
   float alpha;
+  int tiles_n;          // workgroup tiles along n
+  int64_t tiles;        // workgroup tiles of a slice
 };
 
-template <bool kNT>
-__global__ __launch_bounds__(kGemmBlock) void gemm_f32_k(const GemmArgs g) {
-  __shared__ __attribute__((aligned(16))) float as[kGK][kGM + 4];
-  __shared__ __attribute__((aligned(16))) float bs[kGK][kGN + 4];
-  const int64_t slice = blockIdx.z;
+// Columns 8 j + 4 h + (0..3) of lane half h to columns 2 i + h of products
+// i = 0..3 of the eight (v_permlane32_swap exchanges the first's high half
+// with the second's low half).
+__device__ __forceinline__ float4 product_order(float4 v) {
+  const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v.x), __float_as_uint(v.y), false, false);
+  const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(v.z), __float_as_uint(v.w), false, false);
+  return make_float4(__uint_as_float(p[0]), __uint_as_float(q[0]), __uint_as_float(p[1]), __uint_as_float(q[1]));
+}
+
+// Four consecutive floats: one 16-byte read, or four.
+template <bool kVec>
+__device__ __forceinline__ float4 load4(const float* p) {
+  if constexpr (kVec) return *reinterpret_cast<const float4*>(p);
+  return make_float4(p[0], p[1], p[2], p[3]);
+}
+
+// Wave tiles of 32 TM x 32 TN outputs. kSplitK: the workgroup's 4 waves take
+// one tile's k in four runs (summed in wave order through LDS); else four
+// tiles, two by two. kKC: columns of k held per span. kVecA / kVecB: the
+// operand's rows allow 16-byte reads (kVecB for gemm_nt).
+template <bool kNT, int TM, int TN, bool kSplitK, int kKC, bool kVecA, bool kVecB>
+__global__ __launch_bounds__(kGemmWaves * kWave) void gemm_f32_k(const GemmArgs g) {
+  constexpr int kJ = kKC / 8;
+  __shared__ float part[kSplitK ? kGemmWaves * TN * 16 * kWave : 1];
+  const int lane = static_cast<int>(threadIdx.x) % kWave, wave = wave_in_block();
+  const int hl = lane >> 5, c = lane & 31;
+  const unsigned id = xcd_block(blockIdx.x, gridDim.x);
+  const int64_t slice = id / g.tiles;
+  const int tile = static_cast<int>(id - slice * g.tiles);
+  const int tm = tile / g.tiles_n, tn = tile - tm * g.tiles_n;
   const float* A = g.a + slice * g.sa;
   const float* B = g.b + slice * g.sb;
   float* C = g.c + slice * g.sc;
-  const int64_t m0 = static_cast<int64_t>(blockIdx.y) * kGM, n0 = static_cast<int64_t>(blockIdx.x) * kGN;
-  const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-  float acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
+  const int64_t m0 = (kSplitK ? static_cast<int64_t>(tm) : 2 * static_cast<int64_t>(tm) + wave / 2) * kGemmTile * TM;
+  const int64_t n0 = (kSplitK ? static_cast<int64_t>(tn) : 2 * static_cast<int64_t>(tn) + wave % 2) * kGemmTile * TN;
+  if (!kSplitK && (m0 >= g.m || n0 >= g.n)) return;  // no barrier on this path
+  int64_t k = 0, ke = g.k;
+  if (kSplitK) {
+    const int64_t run = (g.k + 8 * kGemmWaves - 1) / (8 * kGemmWaves) * 8;
+    k = run * wave < g.k ? run * wave : g.k;
+    ke = k + run < g.k ? k + run : g.k;
   }
-  for (int64_t k0 = 0; k0 < g.k; k0 += kGK) {
+  // rows and columns past the end repeat the last one; their sums are not stored
+  const float* ap[TM];
+  const float* bp[TN];
 #pragma unroll
-    for (int i = 0; i < kGM * kGK / kGemmBlock; ++i) {
-      const int id = static_cast<int>(threadIdx.x) + kGemmBlock * i;
-      const int r = id / kGK, kk = id % kGK;
-      const int64_t row = m0 + r, kc = k0 + kk;
-      as[kk][r] = row < g.m && kc < g.k ? A[row * g.lda + kc] : 0.0f;
-    }
+  for (int t = 0; t < TM; ++t) {
+    const int64_t row = m0 + kGemmTile * t + c;
+    ap[t] = A + (row < g.m ? row : g.m - 1) * g.lda;
+  }
+#pragma unroll
+  for (int t = 0; t < TN; ++t) {
+    const int64_t col = n0 + kGemmTile * t + c;
+    bp[t] = kNT ? B + (col < g.n ? col : g.n - 1) * g.ldb : B + (col < g.n ? col : g.n - 1);
+  }
+  auto load_b = [&](int t, int64_t k8) -> float4 {
     if constexpr (kNT) {
-#pragma unroll
-      for (int i = 0; i < kGN * kGK / kGemmBlock; ++i) {
-        const int id = static_cast<int>(threadIdx.x) + kGemmBlock * i;
-        const int r = id / kGK, kk = id % kGK;
-        const int64_t col = n0 + r, kc = k0 + kk;
-        bs[kk][r] = col < g.n && kc < g.k ? B[col * g.ldb + kc] : 0.0f;
-      }
+      return load4<kVecB>(bp[t] + k8 + 4 * hl);
     } else {
-#pragma unroll
-      for (int i = 0; i < kGN * kGK / kGemmBlock; ++i) {
-        const int id = static_cast<int>(threadIdx.x) + kGemmBlock * i;
-        const int kk = id / kGN, cc = id % kGN;
-        const int64_t col = n0 + cc, kc = k0 + kk;
-        bs[kk][cc] = col < g.n && kc < g.k ? B[kc * g.ldb + col] : 0.0f;
-      }
+      const float* p = bp[t] + (k8 + hl) * g.ldb;  // already in the products' order
+      return make_float4(p[0], p[2 * g.ldb], p[4 * g.ldb], p[6 * g.ldb]);
     }
-    __syncthreads();
+  };
+  f32x16 acc[TM][TN];
 #pragma unroll
-    for (int kk = 0; kk < kGK; ++kk) {
-      const u32x4 av = *reinterpret_cast<const u32x4*>(&as[kk][4 * ty]);
-      const u32x4 bv = *reinterpret_cast<const u32x4*>(&bs[kk][4 * tx]);
-      const float a4[4] = {__uint_as_float(av.x), __uint_as_float(av.y), __uint_as_float(av.z), __uint_as_float(av.w)};
-      const float b4[4] = {__uint_as_float(bv.x), __uint_as_float(bv.y), __uint_as_float(bv.z), __uint_as_float(bv.w)};
+  for (int i = 0; i < TM; ++i) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+    for (int j = 0; j < TN; ++j) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_fmaf(a4[i], b4[j], acc[i][j]);
-      }
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
     }
-    __syncthreads();
   }
+  auto multiply = [&](const float4 (&xs)[TM], const float4 (&ys)[TN]) {
+    float4 x[TM], y[TN];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int64_t row = m0 + 4 * ty + i;
-    if (row >= g.m) continue;
+    for (int t = 0; t < TM; ++t) x[t] = product_order(xs[t]);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int64_t col = n0 + 4 * tx + j;
-      if (col < g.n) C[row * g.ldc + col] = g.alpha * acc[i][j];
+    for (int t = 0; t < TN; ++t) y[t] = kNT ? product_order(ys[t]) : ys[t];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[i].x, y[j].x, acc[i][j], 0, 0, 0);
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[i].y, y[j].y, acc[i][j], 0, 0, 0);
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[i].z, y[j].z, acc[i][j], 0, 0, 0);
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[i].w, y[j].w, acc[i][j], 0, 0, 0);
+      }
+    }
+  };
+  float4 x[kJ][TM], y[kJ][TN], xn[kJ][TM], yn[kJ][TN];
+  auto load_span = [&](int64_t at, float4 (&xs)[kJ][TM], float4 (&ys)[kJ][TN]) {
+#pragma unroll
+    for (int j = 0; j < kJ; ++j) {
+#pragma unroll
+      for (int t = 0; t < TM; ++t) xs[j][t] = load4<kVecA>(ap[t] + at + 8 * j + 4 * hl);
+#pragma unroll
+      for (int t = 0; t < TN; ++t) ys[j][t] = load_b(t, at + 8 * j);
+    }
+  };
+  if (k + kKC <= ke) {
+    load_span(k, x, y);
+    while (k + 2 * kKC <= ke) {
+      load_span(k + kKC, xn, yn);
+      __builtin_amdgcn_sched_barrier(0);  // the next span's reads go out before this span's products
+#pragma unroll
+      for (int j = 0; j < kJ; ++j) multiply(x[j], y[j]);
+#pragma unroll
+      for (int j = 0; j < kJ; ++j) {
+#pragma unroll
+        for (int t = 0; t < TM; ++t) x[j][t] = xn[j][t];
+#pragma unroll
+        for (int t = 0; t < TN; ++t) y[j][t] = yn[j][t];
+      }
+      k += kKC;
+    }
+#pragma unroll
+    for (int j = 0; j < kJ; ++j) multiply(x[j], y[j]);
+    k += kKC;
+  }
+  for (; k + 8 <= ke; k += 8) {
+#pragma unroll
+    for (int t = 0; t < TM; ++t) x[0][t] = load4<kVecA>(ap[t] + k + 4 * hl);
+#pragma unroll
+    for (int t = 0; t < TN; ++t) y[0][t] = load_b(t, k);
+    multiply(x[0], y[0]);
+  }
+  if (k < ke) {  // the last columns one by one, zeros past them on both sides
+    auto tail = [&](const float* p, int64_t step, int64_t first, int64_t apart) {
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int64_t at = k + first + e * apart;
+        v[e] = at < ke ? p[at * step] : 0.0f;
+      }
+      return make_float4(v[0], v[1], v[2], v[3]);
+    };
+#pragma unroll
+    for (int t = 0; t < TM; ++t) x[0][t] = tail(ap[t], 1, 4 * hl, 1);
+#pragma unroll
+    for (int t = 0; t < TN; ++t) y[0][t] = kNT ? tail(bp[t], 1, 4 * hl, 1) : tail(bp[t], g.ldb, hl, 2);
+    multiply(x[0], y[0]);
+  }
+
+  // register r of lane half h: row 8 (r / 4) + 4 h + r % 4, column c
+  if constexpr (kSplitK) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      if (i > 0) __syncthreads();  // part is read
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) part[((wave * TN + j) * 16 + r) * kWave + lane] = acc[i][j][r];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int64_t col = n0 + kGemmTile * j + c;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {  // this wave's quarter of the registers
+          float sum = part[(j * 16 + 4 * wave + r) * kWave + lane];
+#pragma unroll
+          for (int w = 1; w < kGemmWaves; ++w) sum += part[((w * TN + j) * 16 + 4 * wave + r) * kWave + lane];
+          const int64_t row = m0 + kGemmTile * i + 8 * wave + 4 * hl + r;
+          if (row < g.m && col < g.n) C[row * g.ldc + col] = g.alpha * sum;
+        }
+      }
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int64_t col = n0 + kGemmTile * j + c;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int64_t row = m0 + kGemmTile * i + 8 * (r / 4) + 4 * hl + r % 4;
+          if (row < g.m && col < g.n) C[row * g.ldc + col] = g.alpha * acc[i][j][r];
+        }
+      }
     }
   }
 }
@@ -208,6 +332,30 @@ __global__ __launch_bounds__(kWave) void scatter_rows_once_k(float* dst, const i
 // than the walk, whose one dependent load and store a row takes 0.28 us.
 constexpr int64_t kScatterScanRows = 65536;
 
+constexpr int64_t kGemmGrid = int64_t{1} << 23;  // workgroups a launch (of 256 threads, below 2^32 in all)
+
+// The four forms a product takes: 64 x 64 or 32 x 32 wave tiles with k whole,
+// 64 x 32 or 32 x 32 tiles with k over the workgroup's four waves.
+enum class GemmForm { kWide, kWhole32, kSplit64, kSplit32 };
+
+// Products of at most this many columns are summed in column order as one
+// chain; longer ones as four.
+constexpr int64_t kGemmChain = 256;
+
+template <bool kNT, bool kVecA, bool kVecB>
+void launch_gemm(const GemmArgs& g, unsigned grid, GemmForm form, hipStream_t st) {
+  constexpr int kThreads = kGemmWaves * kWave;
+  if (form == GemmForm::kWide) {
+    gemm_f32_k<kNT, 2, 2, false, 8, kVecA, kVecB><<<grid, kThreads, 0, st>>>(g);
+  } else if (form == GemmForm::kWhole32) {
+    gemm_f32_k<kNT, 1, 1, false, 32, kVecA, kVecB><<<grid, kThreads, 0, st>>>(g);
+  } else if (form == GemmForm::kSplit64) {
+    gemm_f32_k<kNT, 2, 1, true, 16, kVecA, kVecB><<<grid, kThreads, 0, st>>>(g);
+  } else {
+    gemm_f32_k<kNT, 1, 1, true, 32, kVecA, kVecB><<<grid, kThreads, 0, st>>>(g);
+  }
+}
+
 int gemm_entry(const char* what, bool nt, void* stream, int64_t m, int64_t n, int64_t k, float alpha, const float* a,
                int64_t lda, int64_t stride_a, const float* b, int64_t ldb, int64_t stride_b, float* c, int64_t ldc,
                int64_t stride_c, int64_t batch) {
@@ -216,15 +364,49 @@ int gemm_entry(const char* what, bool nt, void* stream, int64_t m, int64_t n, in
   UOCR_REQUIRE(a != nullptr && b != nullptr && c != nullptr, what, "null pointer");
   UOCR_REQUIRE(lda >= k && ldc >= n && ldb >= (nt ? k : n), what, "a leading dimension is below the row width");
   UOCR_REQUIRE(stride_a >= 0 && stride_b >= 0 && stride_c >= 0, what, "strides must be >= 0");
-  const int64_t gx = (n + kGN - 1) / kGN, gy = (m + kGM - 1) / kGM;
-  UOCR_REQUIRE(gx < (int64_t{1} << 31) && gy < 65536 && batch < 65536, what, "grid too large");
-  GemmArgs g{a, b, c, m, n, k, lda, ldb, ldc, stride_a, stride_b, stride_c, alpha};
-  const dim3 grid(static_cast<unsigned>(gx), static_cast<unsigned>(gy), static_cast<unsigned>(batch));
+  UOCR_REQUIRE((m + 63) / 64 < 65536 && batch < 65536, what, "grid too large");
   clear_launch_error();
-  if (nt) {
-    gemm_f32_k<true><<<grid, kGemmBlock, 0, as_stream(stream)>>>(g);
-  } else {
-    gemm_f32_k<false><<<grid, kGemmBlock, 0, as_stream(stream)>>>(g);
+  const auto up = [](int64_t x, int64_t d) { return (x + d - 1) / d; };
+  // Short k: the wide tiles read least a product, where there are enough of
+  // them to give every SIMD one (us, wide / 32 x 32: 10 x 1003 x 1520 k 96
+  // 47 / 61, 16 x 512 x 512 k 128 17 / 24, 16 x 257 x 257 k 96 11.6 / 9.5).
+  // Long k over four waves, with the larger tile once it gives every CU a
+  // workgroup (whole / 64 x 32 / 32 x 32: 10 x 1003 x 96 k 1520 94 / 46 / 56,
+  // 4096 x 64 k 1280 38 / 17.8 / 12.7). A thread per 4 x 4 outputs over
+  // operands staged in LDS, the form before these, took 67, 31, 14.1, 272 and
+  // 161 us on the same five. Outputs past 2^34 take the wide tiles, whose
+  // grid then still fits.
+  const int64_t wide = up(m, 64) * up(n, 64);
+  const GemmForm form = wide >= kGemmGrid / 2 || (k <= kGemmChain && wide * batch >= 1024) ? GemmForm::kWide
+                        : k <= kGemmChain                                              ? GemmForm::kWhole32
+                        : up(m, 64) * up(n, 32) * batch >= 256                         ? GemmForm::kSplit64
+                                                                                       : GemmForm::kSplit32;
+  const int64_t tile_m = form == GemmForm::kWide ? 128 : form == GemmForm::kSplit32 ? 32 : 64;
+  const int64_t tile_n = form == GemmForm::kWide ? 128 : form == GemmForm::kWhole32 ? 64 : 32;
+  const int64_t tiles_n = up(n, tile_n), tiles = up(m, tile_m) * tiles_n;
+  UOCR_REQUIRE(tiles < kGemmGrid, what, "grid too large");
+  const auto rows16 = [](const float* p, int64_t ld, int64_t stride, int64_t slices) {
+    return aligned16(p) && ld % 4 == 0 && (slices == 1 || stride % 4 == 0);
+  };
+  const bool va = rows16(a, lda, stride_a, batch), vb = nt && rows16(b, ldb, stride_b, batch);
+  const int64_t per = kGemmGrid / tiles;  // slices a launch
+  for (int64_t s = 0; s < batch; s += per) {
+    const int64_t count = batch - s < per ? batch - s : per;
+    const GemmArgs g{a + s * stride_a, b + s * stride_b, c + s * stride_c, m, n, k, lda, ldb, ldc,
+                     stride_a, stride_b, stride_c, alpha, static_cast<int>(tiles_n), tiles};
+    const unsigned grid = static_cast<unsigned>(tiles * count);
+    const hipStream_t st = as_stream(stream);
+    if (nt) {
+      if (va && vb) {
+        launch_gemm<true, true, true>(g, grid, form, st);
+      } else {
+        launch_gemm<true, false, false>(g, grid, form, st);
+      }
+    } else if (va) {
+      launch_gemm<false, true, false>(g, grid, form, st);
+    } else {
+      launch_gemm<false, false, false>(g, grid, form, st);
+    }
   }
   return check_launch(what);
 }

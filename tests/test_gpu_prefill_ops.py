@@ -111,3 +111,60 @@ def test_scatter_add_rows_in_order(backend, rows, cols, pick):
             want[idx[i]] = want[idx[i]] + (np.float32(w[i]) * part[i]).astype(np.float32)
         assert np.array_equal(host_f32(dst).view(np.uint32), want.view(np.uint32)), f"shift {shift}"
         assert torch.count_nonzero(buf[:shift]) == 0 and torch.count_nonzero(buf[shift + count * cols:]) == 0
+
+
+# (m, n, k, batch): each form (wide tiles with short k, k over the waves with
+# 64- and 32-row tiles) at its tile edges and at k of less than a run, whole
+# spans and remainders; pad: extra columns in every leading dimension and
+# between slices (odd: no 16-byte reads).
+@pytest.mark.parametrize("m,n,k,batch", [(2049, 2047, 33, 1), (193, 130, 160, 90), (64, 64, 8, 1100), (257, 257, 96, 16),
+                                         (1003, 96, 517, 3), (33, 31, 7, 2), (65, 64, 1283, 1), (1, 1, 129, 5),
+                                         (4096, 64, 1280, 1)])
+@pytest.mark.parametrize("pad", [0, 1, 4])
+def test_gemm_forms(backend, m, n, k, batch, pad):
+    def operand(seed, r, c):
+        ld, st = c + pad, r * (c + pad) + pad
+        flat = dev_f32(normal(seed, batch * st))
+        return flat, ld, st, torch.as_strided(flat, (batch, r, c), (st, ld, 1))
+
+    a, lda, sa, av = operand(540, m, k)
+    c_flat = torch.full((batch * (m * (n + pad) + pad),), float("nan"), device="cuda")
+    ldc, sc = n + pad, m * (n + pad) + pad
+    cv = torch.as_strided(c_flat, (batch, m, n), (sc, ldc, 1))
+    for nt in (True, False):
+        b, ldb, sb, bv = operand(541, n, k) if nt else operand(542, k, n)
+        if nt:
+            backend.gemm_nt(m, n, k, 0.5, a, lda, sa, b, ldb, sb, c_flat, ldc, sc, batch)
+        else:
+            backend.gemm_nn(m, n, k, a, lda, sa, b, ldb, sb, c_flat, ldc, sc, batch)
+        alpha = 0.5 if nt else 1.0
+        for s in range(0, batch, max(1, batch // 3)):
+            x, y = av[s].double(), (bv[s].t() if nt else bv[s]).double().contiguous()
+            want, bound = alpha * (x @ y), alpha * (x.abs() @ y.abs()) * (k + 2) * 2.0 ** -24
+            assert torch.all((cv[s].double() - want).abs() <= bound + 1e-37), f"nt {nt} slice {s}"
+        c_flat.fill_(float("nan"))
+
+
+def test_gemm_special_values(backend):
+    """Infinities and NaN reach exactly the outputs they meet; products and
+    sums below the normal range are kept; k = 0 gives zeros."""
+    m, n, k = 70, 40, 140
+    a, b = normal(550, (m, k)), normal(551, (n, k))
+    a[3, 139], a[5, 0], b[7, 64], a[9, 3], b[9, 3] = np.inf, np.nan, -np.inf, np.inf, 0.0
+    a[11], b[11] = 0.0, 0.0
+    a[11, 5], b[11, 5] = 2.0 ** -100, 2.0 ** -40
+    with np.errstate(invalid="ignore"):
+        want = (a.astype(np.float64) @ b.T.astype(np.float64)).astype(np.float32)
+    c = torch.empty(m, n, device="cuda")
+    for nt in (True, False):
+        if nt:
+            backend.gemm_nt(m, n, k, 1.0, dev_f32(a), k, 0, dev_f32(b), k, 0, c, n, 0)
+        else:
+            backend.gemm_nn(m, n, k, dev_f32(a), k, 0, dev_f32(np.ascontiguousarray(b.T)), n, 0, c, n, 0)
+        got = host_f32(c)
+        finite = np.isfinite(want)
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+        assert np.max(np.abs(got[finite] - want[finite])) <= 1e-5 * np.max(np.abs(want[finite]))
+        assert got[11, 11] == np.float32(2.0 ** -140)
+    backend.gemm_nt(m, n, 0, 1.0, dev_f32(a), k, 0, dev_f32(b), k, 0, c, n, 0)
+    assert torch.count_nonzero(c) == 0
