@@ -4,31 +4,31 @@
 // ops.cu:268-287, which rounds x to bf16 in its own pass and calls a bf16
 // cuBLAS GEMM with fp32 compute, then adds the bias).
 //
-// Both operands are k-contiguous (x rows, w rows), so one tile layout serves
-// both. A workgroup of 4 waves computes a 128 x 128 tile of y; wave (wm, wn)
-// owns a 64 x 64 quarter as 2 x 2 v_mfma_f32_32x32x16_bf16 tiles. The k
-// loop steps 64 at a time through two LDS buffers. Tile rows are 8 chunks of
-// 8 bf16 (16 bytes); a chunk's slot is XOR-swizzled by the row so that the
-// rows one operand read spans fall on different banks (slot() below). Two kernels:
-//   * x already bf16 and k a multiple of 64: both tiles go from memory
-//     straight into LDS (16-byte global_load_lds, each lane's chunk picked so
-//     that it lands in its swizzled slot), the next step's loads in flight
-//     while the current step's 16 matrix products run;
-//   * otherwise (fp32 x, or k not a multiple of 64): chunks staged through
-//     registers, x rounded to bf16 with the hardware's nearest-even
-//     conversion on the way, chunks past k zero-filled; a k that is not a
-//     multiple of 8 (or unaligned rows) loads element by element.
+// Both operands are k-contiguous (x rows, w rows), so one layout serves both:
+// tile rows in LDS are chunks of 8 bf16 (16 bytes), a chunk's slot XOR-swizzled
+// by its row so that the rows one operand read spans fall on different banks.
+// Two kernels, both on v_mfma_f32_32x32x16_bf16:
+//   * linear_pipe_k, x already bf16 and k a multiple of 64: the tiles go from
+//     memory straight into LDS (16-byte global_load_lds, each lane's chunk
+//     picked so that it lands in its swizzled slot), one or two steps of k
+//     ahead of the products. Its forms, small tiles to large, are chosen by
+//     the tile count (form_of below);
+//   * linear_staged_k otherwise (fp32 x, or k not a multiple of 64): 128 x 128
+//     tiles of 4 waves, chunks staged through registers, x rounded to bf16
+//     with the hardware's nearest-even conversion on the way, chunks past k
+//     zero-filled; a k that is not a multiple of 8 (or unaligned rows) loads
+//     element by element. A product with few tiles and a long k may split k
+//     over a caller's workspace: each split writes its partial products and
+//     one more launch sums them in split order, then adds the bias.
 // Workgroups are dealt to the 8 XCDs round-robin; each XCD takes a
 // contiguous run of tiles, ordered in groups of 8 tile-rows sweeping the
 // columns, so the tiles resident on one XCD share x rows and w rows in its
 // L2. The bias is added to each finished sum (one fp32 rounding, as the
-// reference's separate bias pass). A product with few tiles and a long k
-// (the vision encoder's convolutions, CLIP's 257-row projections) may split
-// k over a caller's workspace: each split writes its partial products and one
-// more launch sums them in split order, then adds the bias. Products of bf16
-// rows with no epilogue beyond the bias and the add into y, at least 128
-// rows, go to hipBLASLt instead (gemm_library.hip); the tiles take the
-// activation epilogues, the row scatter, fp32 rows and few rows.
+// reference's separate bias pass). Products of bf16 rows with no epilogue
+// beyond the bias and the add into y, at least 128 rows and too many tiles
+// for the small forms, go to hipBLASLt instead (gemm_library.hip).
+
+#include <type_traits>
 
 #include "act_math.hpp"
 #include "common.hpp"
@@ -94,13 +94,16 @@ struct LinearArgs {
   // product followed by an in-place add
   bool accumulate;
   // Non-null: product row r goes to y row row_map[r], dropped when that is
-  // y_rows or more (a scatter of window slots back into a grid); the
-  // TM x 128 kernels only, no split.
+  // y_rows or more (a scatter of window slots back into a grid); linear_pipe_k
+  // only.
   const int64_t* row_map;
   int64_t y_rows;
   // the activation epilogues' output: y16 = bf16(act(sum + bias)), no split,
   // no accumulate
   uint16_t* y16;
+  // n a multiple of 4 and bias, y and y16 allow 16-byte (y16: 8-byte) accesses
+  bool vec;
+  int runs;  // linear_staged_k: runs of k, 1 with a split
 };
 
 // What the epilogue writes: the fp32 sums, or an MLP's activation of them
@@ -109,9 +112,13 @@ struct LinearArgs {
 enum class Epi { kPlain, kGeluBf16, kQuickGeluBf16 };
 
 template <Epi kEpi>
+__device__ __forceinline__ float activate(float v) {
+  return kEpi == Epi::kGeluBf16 ? gelu_f<10>(v) : quick_gelu_f(v);
+}
+
+template <Epi kEpi>
 __device__ __forceinline__ void store_act(const LinearArgs& a, int64_t row, int64_t col, float v) {
-  v = kEpi == Epi::kGeluBf16 ? gelu_f<10>(v) : quick_gelu_f(v);
-  a.y16[row * a.n + col] = f32_to_bf16(v);
+  a.y16[row * a.n + col] = f32_to_bf16(activate<kEpi>(v));
 }
 
 // 16 elements of one output column, product rows row0 + 8 (r / 4) + r % 4
@@ -143,14 +150,13 @@ struct Work {
   int split, k_begin, k_end;
 };
 
-template <int kTileRows = kTileM>
 __device__ __forceinline__ Work work_of(const LinearArgs& a) {
   const int tiles = a.tiles_m * a.tiles_n;
   const int split = static_cast<int>(blockIdx.x) / tiles;
   int tm, tn;
   tile_of(static_cast<int>(blockIdx.x) - split * tiles, a.tiles_m, a.tiles_n, tm, tn);
   const int kb = split * a.k_len;
-  return {static_cast<int64_t>(tm) * kTileRows, static_cast<int64_t>(tn) * kTileN, split, kb,
+  return {static_cast<int64_t>(tm) * kTileM, static_cast<int64_t>(tn) * kTileN, split, kb,
           a.k - kb < a.k_len ? a.k : kb + a.k_len};
 }
 
@@ -248,15 +254,13 @@ __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast
 
 // The 16 matrix products of one 64-wide k step of a wave's 64 x 64 quarter
 // from the tiles in LDS. The operand reads of slice kk + 1 go out one
-// between each two products of slice kk, and `issue` (the next step's
-// memory-to-LDS loads, kIssued instructions, or nothing) among the first
-// slice's products: a wave never waits on LDS with products it could have
-// issued (the group barriers pin that order; left to itself the scheduler
-// bunches the reads and waits for them before the products).
-template <int kIssued, class Issue>
+// between each two products of slice kk: a wave never waits on LDS with
+// products it could have issued (the group barriers pin that order; left to
+// itself the scheduler bunches the reads and waits for them before the
+// products).
 __device__ __forceinline__ void mfma_step(const u32x4* xs, const u32x4* ws, int wm, int wn, int half, int r32,
-                                          f32x16 (&acc)[2][2], Issue issue) {
-  constexpr int kMfma = 0x008, kDsRead = 0x100, kVmemRead = 0x020;
+                                          f32x16 (&acc)[2][2]) {
+  constexpr int kMfma = 0x008, kDsRead = 0x100;
   bf16x8 fa[2][2], fb[2][2];
   auto read = [&](int kk, int b) {
     const int c = 2 * kk + half;
@@ -270,7 +274,6 @@ __device__ __forceinline__ void mfma_step(const u32x4* xs, const u32x4* ws, int 
 #pragma unroll
   for (int kk = 0; kk < kTileK / 16; ++kk) {
     if (kk + 1 < kTileK / 16) read(kk + 1, (kk + 1) & 1);
-    if (kk == 0) issue();
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
 #pragma unroll
@@ -283,53 +286,50 @@ __device__ __forceinline__ void mfma_step(const u32x4* xs, const u32x4* ws, int 
       for (int q = 0; q < 4; ++q) {
         __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
         __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
-        if (kk == 0 && kIssued > 0) __builtin_amdgcn_sched_group_barrier(kVmemRead, (kIssued + 3) / 4, 0);
       }
     }
     __builtin_amdgcn_sched_barrier(0);
   }
 }
 
-// acc[i][j][r] is y row 8 (r / 4) + 4 half + r % 4 of the 32 x 32 tile,
-// column r32.
-template <Epi kEpi = Epi::kPlain>
-__device__ __forceinline__ void store_tile(const LinearArgs& a, const Work& wk, int wm, int wn, int half, int r32,
-                                           const f32x16 (&acc)[2][2]) {
-  const bool split = a.part != nullptr;
-  float* out = split ? a.part + static_cast<int64_t>(wk.split) * a.m * a.n : a.y;
+// One 32 x 32 product tile into `out`: v[r] is row row0 + 8 (r / 4) + r % 4
+// (row0 the tile's first row + 4 half), column col (of this lane). The bias,
+// the add into y, the row map and the activation apply unless `split`.
+template <Epi kEpi>
+__device__ __forceinline__ void store_frag(const LinearArgs& a, float* out, bool split, int64_t row0, int64_t col,
+                                           const f32x16& v) {
+  if (col >= a.n) return;
   const bool add = !split && a.bias != nullptr;
   const bool accumulate = !split && a.accumulate;
+  const float bv = add ? a.bias[col] : 0.0f;
+  if constexpr (kEpi != Epi::kPlain) {
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int64_t col = wk.n0 + 64 * wn + 32 * j + r32;
-    if (col >= a.n) continue;
-    const float bv = add ? a.bias[col] : 0.0f;
+    for (int r = 0; r < 16; ++r) {
+      const int64_t row = row0 + 8 * (r / 4) + (r % 4);
+      if (row < a.m) store_act<kEpi>(a, row, col, add ? v[r] + bv : v[r]);
+    }
+    return;
+  }
+  if (a.row_map != nullptr) {
+    float val[16];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int64_t row0 = wk.m0 + 64 * wm + 32 * i + 4 * half;
-      if constexpr (kEpi != Epi::kPlain) {
+    for (int r = 0; r < 16; ++r) val[r] = v[r];
+    store_mapped(a, row0, col, bv, add, val);
+    return;
+  }
+  float* const o = out + row0 * a.n + col;  // element r: row row0 + 8 (r / 4) + r % 4
+  auto live = [&](int r) { return row0 + 8 * (r / 4) + (r % 4) < a.m; };
+  auto off = [&](int r) { return static_cast<int64_t>(8 * (r / 4) + (r % 4)) * a.n; };
+  // accumulate: the 16 y values are requested before the first store (a
+  // load issued after a store could alias it and would wait for it)
+  float base[16];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int64_t row = row0 + 8 * (r / 4) + (r % 4);
-          if (row < a.m) store_act<kEpi>(a, row, col, add ? acc[i][j][r] + bv : acc[i][j][r]);
-        }
-        continue;
-      }
-      float* const o = out + row0 * a.n + col;  // element r: row row0 + 8 (r / 4) + r % 4
-      auto live = [&](int r) { return row0 + 8 * (r / 4) + (r % 4) < a.m; };
-      auto off = [&](int r) { return static_cast<int64_t>(8 * (r / 4) + (r % 4)) * a.n; };
-      // accumulate: the 16 y values are requested before the first store (a
-      // load issued after a store could alias it and would wait for it)
-      float base[16];
+  for (int r = 0; r < 16; ++r) base[r] = accumulate && live(r) ? o[off(r)] : 0.0f;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) base[r] = accumulate && live(r) ? o[off(r)] : 0.0f;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        if (live(r)) {
-          const float v = add ? acc[i][j][r] + bv : acc[i][j][r];
-          o[off(r)] = accumulate ? base[r] + v : v;
-        }
-      }
+  for (int r = 0; r < 16; ++r) {
+    if (live(r)) {
+      const float s = add ? v[r] + bv : v[r];
+      o[off(r)] = accumulate ? base[r] + s : s;
     }
   }
 }
@@ -373,6 +373,20 @@ __global__ __launch_bounds__(kGemmThreads) void linear_staged_k(const LinearArgs
   f32x16 acc[2][2];
   zero(acc);
   const int steps = (wk.k_end - wk.k_begin + kTileK - 1) / kTileK;
+  // a.runs > 1: the k steps in that many runs, as the split forms of
+  // linear_pipe_k sum theirs (the same rows in fp32 and in bf16 then give the
+  // same sums up to the order of the last additions)
+  f32x16 total[2][2];
+  zero(total);
+  int run = 0, run_end = steps / a.runs;
+  auto fold = [&] {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) total[i][j] += acc[i][j];
+    }
+    zero(acc);
+  };
   Staged<kF32X> s;
   auto load = [&](int k0) {
     if constexpr (kRagged) {
@@ -388,169 +402,270 @@ __global__ __launch_bounds__(kGemmThreads) void linear_staged_k(const LinearArgs
     const int buf = t & 1;
     const bool more = t + 1 < steps;
     if (more) load(wk.k_begin + (t + 1) * kTileK);
-    mfma_step<0>(xs[buf], ws[buf], wm, wn, half, r32, acc, [] {});
+    mfma_step(xs[buf], ws[buf], wm, wn, half, r32, acc);
+    if (a.runs > 1 && t + 1 >= run_end) {
+      fold();
+      do {
+        ++run;
+        run_end = static_cast<int>(static_cast<int64_t>(steps) * (run + 1) / a.runs);
+      } while (run + 1 < a.runs && t + 1 >= run_end);
+    }
     if (more) store_step(s, xs[buf ^ 1], ws[buf ^ 1]);
     lds_barrier();
   }
-  store_tile(a, wk, wm, wn, half, r32, acc);
-}
-
-// bf16 x and k a multiple of 64: tiles go straight from memory into LDS.
-// Each wave issues 4 + 4 16-byte global_load_lds per step, each writing 64
-// consecutive chunk slots (lane l to slot base + l) with the chunk that
-// belongs there under the swizzle. Rows past m or n read a valid row (their
-// sums are never stored). The step's loads are waited for with the wave's
-// own vmcnt before the barrier (a fence there would also wait for the next
-// step's loads); the barrier is an s_barrier with a compiler memory clobber.
-__device__ __forceinline__ void dma_step(const LinearArgs& a, int64_t m0, int64_t n0, int k0, u32x4* xs, u32x4* ws,
-                                         int wave, int lane) {
-  const uint16_t* x = static_cast<const uint16_t*>(a.x);
-#pragma unroll
-  for (int i = 0; i < kTileChunks / kGemmThreads; ++i) {
-    const int s0 = (wave * (kTileChunks / kGemmThreads) + i) * kWave;  // wave-uniform
-    const int sl = s0 + lane, row = sl / kRowChunks, c = (sl % kRowChunks) ^ swz(row);
-    const int64_t xr = m0 + row < a.m ? m0 + row : a.m - 1;
-    const int64_t wr = n0 + row < a.n ? n0 + row : a.n - 1;
-    __builtin_amdgcn_global_load_lds(x + xr * a.k + k0 + 8 * c, xs + s0, 16, 0, 0);
-    __builtin_amdgcn_global_load_lds(a.w + wr * a.k + k0 + 8 * c, ws + s0, 16, 0, 0);
-  }
-}
-
-template <int kPending>
-__device__ __forceinline__ void wait_loads_and_barrier() {
-  // s_waitcnt vmcnt(kPending) with the other counters left alone, then the
-  // barrier; the asm's memory clobber keeps LDS accesses on their side.
-  __builtin_amdgcn_s_waitcnt((kPending & 0xF) | (((kPending >> 4) & 3) << 14) | (7 << 4) | (0xF << 8));
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
-template <Epi kEpi>
-__global__ __launch_bounds__(kGemmThreads) void linear_dma_k(const LinearArgs a) {
-  __shared__ u32x4 xs[2][kTileChunks];
-  __shared__ u32x4 ws[2][kTileChunks];
-  const Work wk = work_of(a);
-  const int lane = threadIdx.x & (kWave - 1), wave = wave_in_block();
-  const int wm = wave >> 1, wn = wave & 1;
-  const int half = lane >> 5, r32 = lane & 31;
-  f32x16 acc[2][2];
-  zero(acc);
-  const int steps = (wk.k_end - wk.k_begin) / kTileK;
-  dma_step(a, wk.m0, wk.n0, wk.k_begin, xs[0], ws[0], wave, lane);
-  for (int t = 0; t < steps; ++t) {
-    const int buf = t & 1;
-    wait_loads_and_barrier<0>();  // this step's tiles are in LDS; every wave is done with the other buffer
-    const bool more = t + 1 < steps;
-    mfma_step<2 * kTileChunks / kGemmThreads>(xs[buf], ws[buf], wm, wn, half, r32, acc, [&] {
-      if (more) dma_step(a, wk.m0, wk.n0, wk.k_begin + (t + 1) * kTileK, xs[buf ^ 1], ws[buf ^ 1], wave, lane);
-    });
-  }
-  store_tile<kEpi>(a, wk, wm, wn, half, r32, acc);
-}
-
-// Products of few rows (CLIP's 257, a short prompt), or of too few 128-row
-// tiles to give every CU two: TM x 128 tiles with TM 32 or 64, so that a
-// 257-row product has 9 row tiles instead of 3 (the last of them holding
-// one row), and a [4096, 768] output 384 tiles instead of 192. Wave w of 4
-// owns columns 32 w .. 32 w + 31 of the tile, TM / 32
-// v_mfma_f32_32x32x16_bf16 tiles, its operands read from the same swizzled
-// LDS layout as the 128 x 128 tiles; bf16 x and k a multiple of 64, tiles
-// straight from memory into LDS.
-constexpr int kNarrowM = 32;
-
-template <int TM>
-__device__ __forceinline__ void dma_step_narrow(const LinearArgs& a, int64_t m0, int64_t n0, int k0, u32x4* xs,
-                                                u32x4* ws, int wave, int lane) {
-  const uint16_t* x = static_cast<const uint16_t*>(a.x);
-  constexpr int kXPerWave = TM * kRowChunks / kGemmThreads;  // x tile loads per wave: 1 or 2
-#pragma unroll
-  for (int i = 0; i < kXPerWave; ++i) {
-    const int s0 = (wave * kXPerWave + i) * kWave;
-    const int sl = s0 + lane, row = sl / kRowChunks, c = (sl % kRowChunks) ^ swz(row);
-    const int64_t xr = m0 + row < a.m ? m0 + row : a.m - 1;
-    __builtin_amdgcn_global_load_lds(x + xr * a.k + k0 + 8 * c, xs + s0, 16, 0, 0);
-  }
-#pragma unroll
-  for (int i = 0; i < kTileChunks / kGemmThreads; ++i) {
-    const int s0 = (wave * (kTileChunks / kGemmThreads) + i) * kWave;
-    const int sl = s0 + lane, row = sl / kRowChunks, c = (sl % kRowChunks) ^ swz(row);
-    const int64_t wr = n0 + row < a.n ? n0 + row : a.n - 1;
-    __builtin_amdgcn_global_load_lds(a.w + wr * a.k + k0 + 8 * c, ws + s0, 16, 0, 0);
-  }
-}
-
-template <int TM, Epi kEpi>
-__global__ __launch_bounds__(kGemmThreads) void linear_narrow_k(const LinearArgs a) {
-  constexpr int FI = TM / 32;
-  __shared__ u32x4 xs[2][TM * kRowChunks];
-  __shared__ u32x4 ws[2][kTileChunks];
-  const Work wk = work_of<TM>(a);
-  const int lane = threadIdx.x & (kWave - 1), wave = wave_in_block();
-  const int half = lane >> 5, r32 = lane & 31;
-  f32x16 acc[FI];
-#pragma unroll
-  for (int i = 0; i < FI; ++i) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
-  }
-  const int steps = (wk.k_end - wk.k_begin) / kTileK;
-  dma_step_narrow<TM>(a, wk.m0, wk.n0, wk.k_begin, xs[0], ws[0], wave, lane);
-  for (int t = 0; t < steps; ++t) {
-    const int buf = t & 1;
-    wait_loads_and_barrier<0>();  // this step's tiles are in LDS; every wave is done with the other buffer
-    if (t + 1 < steps) {
-      dma_step_narrow<TM>(a, wk.m0, wk.n0, wk.k_begin + (t + 1) * kTileK, xs[buf ^ 1], ws[buf ^ 1], wave, lane);
-    }
-    bf16x8 fa[4][FI], fb[4];
-#pragma unroll
-    for (int kk = 0; kk < kTileK / 16; ++kk) {
-#pragma unroll
-      for (int i = 0; i < FI; ++i) fa[kk][i] = as_bf16x8(xs[buf][slot(32 * i + r32, 2 * kk + half)]);
-      fb[kk] = as_bf16x8(ws[buf][slot(32 * wave + r32, 2 * kk + half)]);
-    }
-#pragma unroll
-    for (int kk = 0; kk < kTileK / 16; ++kk) {
-#pragma unroll
-      for (int i = 0; i < FI; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[kk][i], fb[kk], acc[i], 0, 0, 0);
-    }
-  }
-  // acc[i][r]: row 32 i + 8 (r / 4) + 4 half + r % 4 of the tile, column
-  // 32 wave + r32
   const bool split = a.part != nullptr;
   float* out = split ? a.part + static_cast<int64_t>(wk.split) * a.m * a.n : a.y;
-  const int64_t col = wk.n0 + 32 * wave + r32;
-  if (col >= a.n) return;
-  const bool add = !split && a.bias != nullptr;
-  const bool accumulate = !split && a.accumulate;
-  const float bv = add ? a.bias[col] : 0.0f;
+  if (a.runs > 1) {
 #pragma unroll
-  for (int i = 0; i < FI; ++i) {
-    const int64_t row0 = wk.m0 + 32 * i + 4 * half;
-    if constexpr (kEpi != Epi::kPlain) {
+    for (int i = 0; i < 2; ++i) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[i][j] = total[i][j];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      store_frag<Epi::kPlain>(a, out, split, wk.m0 + 64 * wm + 32 * i + 4 * half, wk.n0 + 64 * wn + 32 * j + r32,
+                              acc[i][j]);
+    }
+  }
+}
+
+typedef __attribute__((address_space(3))) void* LdsPtr;
+
+// One 16-byte memory-to-LDS load a lane: lane l's bytes go to LDS address
+// lds + 16 l. In assembly because the compiler puts a wait for every
+// outstanding load of the builtin's form before the next LDS read, which
+// takes the next step's loads into this step's time (a 64 x 64 tile's step of
+// 64 columns then lasts a whole memory latency, 0.85 us); the callers wait
+// with counts of their own before they read.
+__device__ __forceinline__ void dma16(uint32_t lds, const char* base, uint32_t off) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
+               : "memory");
+}
+__device__ __forceinline__ void dma16(uint32_t lds, const char* base, uint64_t off) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(base + off)
+               : "memory");
+}
+
+// At most kPending of this wave's memory loads outstanding and all its LDS
+// reads returned; with kBarrier, then the workgroup's barrier.
+template <int kPending, bool kBarrier>
+__device__ __forceinline__ void wait_loads() {
+  if constexpr (kBarrier) {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kPending) : "memory");
+  } else {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kPending) : "memory");
+  }
+}
+
+// A tile of TM x TN outputs by WM x WN x WK waves; kKC columns of k a step,
+// kS steps of tiles in LDS, kS - 1 of them in flight ahead of the products.
+//
+// WK = 1: the WM x WN waves share the tiles, one barrier a step (behind it
+// every wave's loads of the step are in LDS and every wave has read the step
+// before, whose tiles the next loads overwrite).
+//
+// WM = WN = 1: each of the WK waves takes the whole tile over a WK-th of k
+// with tiles of its own: no barrier, no operand read twice, and WK times the
+// loads in flight of a tile that few workgroups share the chip for. The
+// partial sums meet in LDS (rows kP floats apart: the two halves of a wave,
+// four rows apart, write different banks) and are added in pairs.
+//
+// What bounds the small forms is the latency from the first load to the last
+// store and, past that, a CU's 64 bytes a clock from L2: 64 x 896 x 1280
+// 17.7 us by the earlier 32 x 128 tiles (one step's loads waited for a step)
+// to 4.9, 64 x 1280 x 6848 91 to 16.5, 65 x 1024 x 4096 43 to 7.8; the
+// library's best without a workspace 7.6 us at 384 x 896 x 1280 against 6.5,
+// 13.6 at 257 x 1024 x 4096 against 10.9.
+//
+// kFar: row offsets of 64 bits (rows of 2^23 columns or more).
+template <int TM, int TN, int WM, int WN, int WK, int kKC, int kS, bool kFar, Epi kEpi>
+__global__ __launch_bounds__(kWave* WM* WN* WK) void linear_pipe_k(const LinearArgs a) {
+  constexpr int kRC = kKC / 8, kGroup = WM * WN;  // chunks a tile row, waves sharing tiles
+  constexpr int kXLoads = TM * kRC / kWave, kLoads = (TM + TN) * kRC / kWave / kGroup;
+  constexpr int FM = TM / WM / 32, FN = TN / WN / 32;
+  constexpr int kStage = (TM + TN) * kRC;
+  constexpr int kP = TN + 8;
+  constexpr int kTiles = WK * kS * kStage, kSums = WK > 1 ? WK * TM * kP / 4 : 0;
+  static_assert((kXLoads + TN * kRC / kWave) % kGroup == 0 && (kGroup == 1 || WK == 1) && kS >= 2 && kS <= 3);
+  static_assert(4 * kP % 64 == 32);
+  using Off = std::conditional_t<kFar, uint64_t, uint32_t>;
+  __shared__ u32x4 lds[kTiles > kSums ? kTiles : kSums];
+  const int lane = threadIdx.x & (kWave - 1), wave = wave_in_block();
+  const int grp = wave / kGroup, wg = wave % kGroup, wm = wg / WN, wn = wg % WN;
+  const int half = lane >> 5, r32 = lane & 31;
+  int tm, tn;
+  tile_of(static_cast<int>(blockIdx.x), a.tiles_m, a.tiles_n, tm, tn);
+  const int64_t m0 = static_cast<int64_t>(tm) * TM, n0 = static_cast<int64_t>(tn) * TN;
+  const int steps = a.k / kKC;
+  const int first = static_cast<int>(static_cast<int64_t>(steps) * grp / WK);
+  const int n = static_cast<int>(static_cast<int64_t>(steps) * (grp + 1) / WK) - first;
+  const char* const xb = static_cast<const char*>(a.x) + (m0 * a.k + static_cast<int64_t>(first) * kKC) * 2;
+  const char* const wb = reinterpret_cast<const char*>(a.w) + (n0 * a.k + static_cast<int64_t>(first) * kKC) * 2;
+  const int xlast = static_cast<int>(a.m - 1 - m0 < TM ? a.m - 1 - m0 : TM - 1);
+  const int wlast = static_cast<int>(a.n - 1 - n0 < TN ? a.n - 1 - n0 : TN - 1);
+  // 16 rows of 128 (64) bytes span 32 (16) bank groups of 16 bytes, of which
+  // there are 16: the chunk moves with the row where the rows repeat
+  auto swizzle = [](int row) { return kRC == 8 ? (row >> 1) & 7 : (row >> 2) & 3; };
+  // load i of this wave: 64 slots of the x tile, then of the w tile; rows
+  // past m or n read the last one (their sums are never stored)
+  Off off[kLoads];
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const int q = wg * kLoads + i;
+    const bool isx = q < kXLoads;
+    const int s = (isx ? q : q - kXLoads) * kWave + lane, row = s / kRC, c = (s % kRC) ^ swizzle(row);
+    const int last = isx ? xlast : wlast;
+    off[i] = static_cast<Off>(row < last ? row : last) * a.k * 2 + c * 16;
+  }
+  u32x4* const mine = lds + grp * kS * kStage;
+  const uint32_t lds0 =
+      __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((LdsPtr)mine)));
+  auto issue = [&](int t, int buf) {
+    const int64_t at = static_cast<int64_t>(t) * kKC * 2;
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const int q = wg * kLoads + i;
+      dma16(lds0 + (buf * kStage + q * kWave) * 16, (q < kXLoads ? xb : wb) + at, off[i]);
+    }
+  };
+  f32x16 acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i) {
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+    }
+  }
+  auto products = [&](int buf) {
+    const u32x4* xs = mine + buf * kStage;
+    const u32x4* ws = xs + TM * kRC;
+    bf16x8 fa[kRC / 2][FM], fb[kRC / 2][FN];
+#pragma unroll
+    for (int kk = 0; kk < kRC / 2; ++kk) {
+      const int c = 2 * kk + half;
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        const int row = 32 * (wm * FM + i) + r32;
+        fa[kk][i] = as_bf16x8(xs[row * kRC + (c ^ swizzle(row))]);
+      }
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        const int row = 32 * (wn * FN + j) + r32;
+        fb[kk][j] = as_bf16x8(ws[row * kRC + (c ^ swizzle(row))]);
+      }
+    }
+#pragma unroll
+    for (int kk = 0; kk < kRC / 2; ++kk) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+#pragma unroll
+        for (int j = 0; j < FN; ++j) {
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[kk][i], fb[kk][j], acc[i][j], 0, 0, 0);
+        }
+      }
+    }
+  };
+#pragma unroll
+  for (int t = 0; t < kS - 1; ++t) {
+    if (t < n) issue(t, t);
+  }
+  int buf = 0, next = kS - 1, t = 0;
+  for (; t + kS - 1 < n; ++t) {
+    wait_loads<(kS - 2) * kLoads, (kGroup > 1)>();
+    issue(t + kS - 1, next);
+    products(buf);
+    buf = buf + 1 == kS ? 0 : buf + 1;
+    next = next + 1 == kS ? 0 : next + 1;
+  }
+  if (kS == 3 && n > 1) {  // the last step's loads still in flight
+    wait_loads<kLoads, (kGroup > 1)>();
+    products(buf);
+    buf = buf + 1 == kS ? 0 : buf + 1;
+  }
+  if (n > 0) {
+    wait_loads<0, (kGroup > 1)>();
+    products(buf);
+  }
+
+  if constexpr (WK == 1) {
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        store_frag<kEpi>(a, a.y, false, m0 + 32 * (wm * FM + i) + 4 * half, n0 + 32 * (wn * FN + j) + r32, acc[i][j]);
+      }
+    }
+    return;
+  }
+  float* const part = reinterpret_cast<float*>(lds);
+  __syncthreads();  // every wave has read its tiles
+#pragma unroll
+  for (int i = 0; i < FM; ++i) {
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int64_t row = row0 + 8 * (r / 4) + (r % 4);
-        if (row < a.m) store_act<kEpi>(a, row, col, add ? acc[i][r] + bv : acc[i][r]);
+        part[(grp * TM + 32 * i + 8 * (r / 4) + 4 * half + r % 4) * kP + 32 * j + r32] = acc[i][j][r];
       }
-      continue;
     }
+  }
+  __syncthreads();
+  constexpr int kQuads = TN / 4, kThreads = kWave * WK;
+  static_assert(TM * kQuads % kThreads == 0);
+  const bool add = a.bias != nullptr;
+#pragma unroll
+  for (int it = 0; it < TM * kQuads / kThreads; ++it) {
+    const int id = static_cast<int>(threadIdx.x) + kThreads * it, row = id / kQuads, q = id % kQuads;
+    static_assert(WK == 1 || WK == 4);
+    float4 u[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) u[g] = *reinterpret_cast<const float4*>(part + (g * TM + row) * kP + 4 * q);
+    float v[4] = {(u[0].x + u[1].x) + (u[2].x + u[3].x), (u[0].y + u[1].y) + (u[2].y + u[3].y),
+                  (u[0].z + u[1].z) + (u[2].z + u[3].z), (u[0].w + u[1].w) + (u[2].w + u[3].w)};
+    const int64_t at = m0 + row, col = n0 + 4 * q;
+    if (at >= a.m || col >= a.n) continue;
+    int64_t to = at;
     if (a.row_map != nullptr) {
-      float val[16];
-#pragma unroll
-      for (int r = 0; r < 16; ++r) val[r] = acc[i][r];
-      store_mapped(a, row0, col, bv, add, val);
-      continue;
+      to = a.row_map[at];
+      if (to >= a.y_rows) continue;
     }
-    float* const o = out + row0 * a.n + col;
-    auto live = [&](int r) { return row0 + 8 * (r / 4) + (r % 4) < a.m; };
-    auto off = [&](int r) { return static_cast<int64_t>(8 * (r / 4) + (r % 4)) * a.n; };
-    float base[16];
+    const int cols = a.n - col < 4 ? static_cast<int>(a.n - col) : 4;
+    if (a.vec) {
+      if (add) {
+        const float4 b = *reinterpret_cast<const float4*>(a.bias + col);
+        v[0] += b.x;
+        v[1] += b.y;
+        v[2] += b.z;
+        v[3] += b.w;
+      }
+      if constexpr (kEpi != Epi::kPlain) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) base[r] = accumulate && live(r) ? o[off(r)] : 0.0f;
+        for (int e = 0; e < 4; ++e) v[e] = activate<kEpi>(v[e]);
+        *reinterpret_cast<uint2*>(a.y16 + to * a.n + col) = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
+      } else {
+        float4* const o = reinterpret_cast<float4*>(a.y + to * a.n + col);
+        if (a.accumulate) {
+          const float4 y = *o;
+          *o = make_float4(y.x + v[0], y.y + v[1], y.z + v[2], y.w + v[3]);
+        } else {
+          *o = make_float4(v[0], v[1], v[2], v[3]);
+        }
+      }
+    } else {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      if (live(r)) {
-        const float v = add ? acc[i][r] + bv : acc[i][r];
-        o[off(r)] = accumulate ? base[r] + v : v;
+      for (int e = 0; e < 4; ++e) {
+        if (e >= cols) continue;
+        if (add) v[e] += a.bias[col + e];
+        if constexpr (kEpi != Epi::kPlain) {
+          store_act<kEpi>(a, at, col + e, v[e]);
+        } else {
+          float* const o = a.y + to * a.n + col + e;
+          *o = a.accumulate ? *o + v[e] : v[e];
+        }
       }
     }
   }
@@ -570,47 +685,94 @@ __global__ __launch_bounds__(kBlock) void round_bf16_k(const float* __restrict__
   }
 }
 
-// Products of at most this many rows take the 32-row tiles (bf16 x, k a
-// multiple of 64), splitting k below this many of those tiles when k is at
-// least 2048 (measured at 257 rows: k 4096 runs 2.5x faster split 16 ways,
-// k 1024 loses 20-30% split 3-4 ways).
-constexpr int64_t kNarrowRows = 512;
-constexpr int64_t kNarrowSplitBelow = 256;
-// Products of more rows whose 128 x 128 tiles are fewer than this (two
-// workgroups per CU), and that would not split k, take 64 x 128 tiles:
-// twice the workgroups, a shorter tail (the decoder's [4096 <- 1280] -> 1280,
-// 320 tiles: 35.7 -> 32.2 us).
-constexpr int64_t kMediumTilesBelow = 512;
+// The forms of linear_pipe_k. Split forms: four waves over k, a tile to each
+// CU; shared forms: waves over the tile.
+enum class Form { kSplit32, kSplit64x32, kSplit64, kShared64, kShared256, kFar };
+
+// Workgroups the split forms want at most: one a CU. A CU holds one of their
+// workgroups (96 to 147 KB of tiles), so one more tile than this costs a
+// second pass over the chip.
+constexpr int64_t kChipTiles = 256;
+// From this many 64 x 64 tiles the 256 x 128 ones (an eighth of the tiles,
+// half the L2 reads a product) are ahead: 4096 x 2304 x 768 (2304) 34.6
+// against 32.3 us, 2500 x 3072 x 768 (1920) 27.2 against 26.0, 4900 x 768 x
+// 768 (924) and below the other way round.
+constexpr int64_t kShared256Tiles = 1536;
+// Rows of this many columns or more: 256 of them are 2^32 bytes.
+constexpr int64_t kFarColumns = int64_t{1} << 23;
+
+int64_t tiles_of(int64_t m, int64_t n, int64_t tm, int64_t tn) { return ((m + tm - 1) / tm) * ((n + tn - 1) / tn); }
+
+// The smallest tiles that the chip holds at once (us at 16 / 64 / 384 / 900 x
+// 896 x 1280, 32 x 32 / 64 x 32 / 64 x 64 split: 4.5 / 5.2 / 6.6; 4.9 / 6.2 /
+// 8.2; 8.0 / 6.5 / 8.2; 17 / 10.7 / 8.4), past them the shared tiles (900 x
+// 1280 x 896, 300 tiles: 64 x 64 split 12.0, shared 9.6). A rule on m, n and k
+// alone, so that a product has the same sums whatever its epilogue.
+// Up to kChain columns there is little to split, and the sums stay one chain
+// over k in column order.
+constexpr int64_t kChain = 256;
+
+Form form_of(int64_t m, int64_t n, int64_t k) {
+  if (k >= kFarColumns) return Form::kFar;
+  if (k <= kChain) return tiles_of(m, n, 64, 64) < kShared256Tiles ? Form::kShared64 : Form::kShared256;
+  if (tiles_of(m, n, 32, 32) <= kChipTiles) return Form::kSplit32;
+  if (tiles_of(m, n, 64, 32) <= kChipTiles) return Form::kSplit64x32;
+  if (tiles_of(m, n, 64, 64) <= kChipTiles) return Form::kSplit64;
+  return tiles_of(m, n, 64, 64) < kShared256Tiles ? Form::kShared64 : Form::kShared256;
+}
+
+// The runs of k a form sums apart.
+int runs_of(Form form) { return form == Form::kShared64 || form == Form::kShared256 ? 1 : 4; }
+
+// Where the library's larger tiles are the faster ones (us, here / library):
+// past the split forms with a long k (1600 x 768 x 3072, 300 tiles 23.4 /
+// 20.3; 2500 x 768 x 3072 25.3 / 22.2; 1024 x 1280 x 6848 54 / 45) and, with
+// a short one, past two passes of the chip (257 x 4096 x 1024, 320 tiles 10.7
+// / 12.0, 400 x 3584 x 1280 14.9 / 15.7, 577 x 3072 x 1024 12.1 / 13.2, 2500 x
+// 768 x 768, 480 tiles 10.1 / 10.6; 577 x 4096 x 1024, 640 tiles 15.4 / 14.6,
+// 4096 x 768 x 768 14.1 / 13.0). A call into the library is 16 us of host
+// time against 3.3, and a shape's first call times its candidates, which
+// these sizes (a prompt's rows, an expert's share of them) hardly ever repeat.
+// Products narrower than one tile stay with the library too (of 128 rows and
+// more): most of a tile would be padding, and the features the small vision
+// model is held to hang on which side of a bf16 rounding such a sum falls.
+bool library_faster(int64_t m, int64_t n, int64_t k) {
+  const int64_t tiles = tiles_of(m, n, 64, 64);
+  return n < 32 || tiles > 2 * kChipTiles || (tiles > kChipTiles && k > 1280);
+}
+
+template <Epi kEpi>
+void launch_pipe(LinearArgs& a, Form form, hipStream_t st) {
+  auto launch = [&]<int TM, int TN, int WM, int WN, int WK, int kKC, int kS, bool kFar>() {
+    a.tiles_m = static_cast<int>((a.m + TM - 1) / TM);
+    a.tiles_n = static_cast<int>((a.n + TN - 1) / TN);
+    linear_pipe_k<TM, TN, WM, WN, WK, kKC, kS, kFar, kEpi>
+        <<<static_cast<unsigned>(a.tiles_m) * static_cast<unsigned>(a.tiles_n), kWave * WM * WN * WK, 0, st>>>(a);
+  };
+  switch (form) {
+    case Form::kSplit32: launch.template operator()<32, 32, 1, 1, 4, 64, 3, false>(); break;
+    case Form::kSplit64x32: launch.template operator()<64, 32, 1, 1, 4, 64, 3, false>(); break;
+    case Form::kSplit64: launch.template operator()<64, 64, 1, 1, 4, 64, 2, false>(); break;
+    case Form::kShared64: launch.template operator()<64, 64, 2, 2, 1, 64, 3, false>(); break;
+    case Form::kShared256: launch.template operator()<256, 128, 4, 2, 1, 32, 3, false>(); break;
+    case Form::kFar: launch.template operator()<32, 32, 1, 1, 4, 64, 3, true>(); break;
+  }
+}
 
 }  // namespace
 
-// The splits of k worth taking for an m x n x k product: a product of
-// fewer than 64 tiles with k >= 1024 (of 32-row tiles: fewer than 256 with
-// k >= 2048) gets enough workgroups to cover the 256 CUs twice, each split
-// at least 4 steps of 64 columns; any other runs unsplit. (Measured at the
-// vision encoder's shapes: 16-24 tiles with k of 2304-4608 run 1.3-1.9x
-// faster split; 72-234 tiles, or k of 768-1024, lose 5-100% to the partial
-// sums' traffic and the extra launch.)
-int64_t splits_for(int64_t m, int64_t k, int64_t n, bool narrow = false) {
-  const int64_t tile_rows = narrow ? kNarrowM : kTileM;
-  const int64_t tiles = ((m + tile_rows - 1) / tile_rows) * ((n + kTileN - 1) / kTileN);
-  if (tiles >= (narrow ? kNarrowSplitBelow : 64) || k < (narrow ? 32 : 16) * kTileK) return 1;
+// The splits of k worth taking for an m x n x k product on the staged tiles:
+// a product of fewer than 64 tiles with k >= 1024 gets enough workgroups to
+// cover the 256 CUs twice, each split at least 4 steps of 64 columns; any
+// other runs unsplit. (Measured at the vision encoder's shapes: 16-24 tiles
+// with k of 2304-4608 run 1.3-1.9x faster split; 72-234 tiles, or k of
+// 768-1024, lose 5-100% to the partial sums' traffic and the extra launch.)
+int64_t splits_for(int64_t m, int64_t k, int64_t n) {
+  const int64_t tiles = ((m + kTileM - 1) / kTileM) * ((n + kTileN - 1) / kTileN);
+  if (tiles >= 64 || k < 16 * kTileK) return 1;
   int64_t s = (512 + tiles - 1) / tiles;
   s = s < k / (4 * kTileK) ? s : k / (4 * kTileK);
   return s < 32 ? s : 32;
-}
-
-// The bf16-x kernels that read their tiles straight into LDS (k a multiple
-// of 64, x and w 16-byte aligned).
-template <Epi kEpi>
-void launch_tiles(const LinearArgs& a, unsigned grid, hipStream_t st, bool narrow, bool medium) {
-  if (narrow) {
-    linear_narrow_k<kNarrowM, kEpi><<<grid, kGemmThreads, 0, st>>>(a);
-  } else if (medium) {
-    linear_narrow_k<2 * kNarrowM, kEpi><<<grid, kGemmThreads, 0, st>>>(a);
-  } else {
-    linear_dma_k<kEpi><<<grid, kGemmThreads, 0, st>>>(a);
-  }
 }
 
 int linear_entry(const char* what, void* stream, const void* x, bool f32x, int64_t m, int64_t k, const uint16_t* w,
@@ -622,50 +784,44 @@ int linear_entry(const char* what, void* stream, const void* x, bool f32x, int64
   UOCR_REQUIRE(k >= 1 && k < (int64_t{1} << 30), what, "k must be in [1, 2^30)");
   UOCR_REQUIRE(x != nullptr && w != nullptr && (epi == Epi::kPlain ? y != nullptr : y16 != nullptr), what,
                "null x, w or y");
+  const bool ragged = k % 8 != 0 || !aligned16(x) || !aligned16(w);
+  const bool pipe = !ragged && !f32x && k % kTileK == 0;
   // products of bf16 rows with no epilogue beyond the bias (and the add
-  // into y) go to the BLAS library when it takes them
-  if (!f32x && epi == Epi::kPlain && row_map == nullptr) {
+  // into y) go to the BLAS library where it is the faster and takes them
+  if (!f32x && epi == Epi::kPlain && row_map == nullptr && (!pipe || library_faster(m, n, k))) {
     const int st =
         library_linear_bf16(what, as_stream(stream), static_cast<const uint16_t*>(x), m, k, w, n, bias, y, accumulate);
     if (st != kLibraryDeclined) return st;
   }
-  const bool ragged = k % 8 != 0 || !aligned16(x) || !aligned16(w);
-  const bool dma = !ragged && !f32x && k % kTileK == 0;
-  const int64_t tiles128 = ((m + kTileM - 1) / kTileM) * ((n + kTileN - 1) / kTileN);
-  const bool narrow = dma && m <= kNarrowRows;
-  // 64-row tiles where the 128-row ones are too few and would not be split
-  // (and always with a row map)
-  const bool medium = dma && !narrow &&
-                      (row_map != nullptr ||
-                       (tiles128 < kMediumTilesBelow && (workspace == nullptr || splits_for(m, k, n) == 1)));
-  const int64_t tile_rows = narrow ? kNarrowM : medium ? 2 * kNarrowM : kTileM;
-  const int64_t tiles_m = (m + tile_rows - 1) / tile_rows, tiles_n = (n + kTileN - 1) / kTileN;
-  UOCR_REQUIRE(tiles_m * tiles_n < (int64_t{1} << 31), what, "too many tiles");
+  UOCR_REQUIRE(tiles_of(m, n, 32, 32) < (int64_t{1} << 31), what, "too many tiles");
+  LinearArgs a{x, w, bias, y, m, n, static_cast<int>(k), 0, 0, static_cast<int>(k), nullptr, accumulate, row_map,
+               y_rows, y16, n % 4 == 0 && (bias == nullptr || aligned16(bias)) && aligned16(y) && aligned16(y16), 1};
+  clear_launch_error();
+  const hipStream_t st = as_stream(stream);
+  if (pipe) {
+    const Form form = form_of(m, n, k);
+    if (epi == Epi::kGeluBf16) {
+      launch_pipe<Epi::kGeluBf16>(a, form, st);
+    } else if (epi == Epi::kQuickGeluBf16) {
+      launch_pipe<Epi::kQuickGeluBf16>(a, form, st);
+    } else {
+      launch_pipe<Epi::kPlain>(a, form, st);
+    }
+    return check_launch(what);
+  }
   // split k into the workspace when it holds the partial products
-  int64_t splits =
-      workspace != nullptr && !medium && row_map == nullptr && epi == Epi::kPlain ? splits_for(m, k, n, narrow) : 1;
+  int64_t splits = workspace != nullptr ? splits_for(m, k, n) : 1;
   if (splits > 1 && workspace_floats < splits * m * n) splits = 1;
   const int64_t k_len = splits > 1 ? (k / splits + kTileK - 1) / kTileK * kTileK : k;
   splits = (k + k_len - 1) / k_len;
+  const int64_t tiles_m = (m + kTileM - 1) / kTileM, tiles_n = (n + kTileN - 1) / kTileN;
   UOCR_REQUIRE(tiles_m * tiles_n * splits < (int64_t{1} << 31), what, "too many tiles");
-  LinearArgs a{x,
-               w,
-               bias,
-               y,
-               m,
-               n,
-               static_cast<int>(k),
-               static_cast<int>(tiles_m),
-               static_cast<int>(tiles_n),
-               static_cast<int>(k_len),
-               splits > 1 ? workspace : nullptr,
-               accumulate,
-               row_map,
-               y_rows,
-               y16};
+  a.tiles_m = static_cast<int>(tiles_m);
+  a.tiles_n = static_cast<int>(tiles_n);
+  a.k_len = static_cast<int>(k_len);
+  a.part = splits > 1 ? workspace : nullptr;
+  if (splits == 1) a.runs = runs_of(form_of(m, n, k));
   const unsigned grid = static_cast<unsigned>(tiles_m * tiles_n * splits);
-  clear_launch_error();
-  const hipStream_t st = as_stream(stream);
   if (ragged) {
     if (f32x) {
       linear_staged_k<true, true><<<grid, kGemmThreads, 0, st>>>(a);
@@ -674,12 +830,6 @@ int linear_entry(const char* what, void* stream, const void* x, bool f32x, int64
     }
   } else if (f32x) {
     linear_staged_k<true, false><<<grid, kGemmThreads, 0, st>>>(a);
-  } else if (epi == Epi::kGeluBf16) {
-    launch_tiles<Epi::kGeluBf16>(a, grid, st, narrow, medium);
-  } else if (epi == Epi::kQuickGeluBf16) {
-    launch_tiles<Epi::kQuickGeluBf16>(a, grid, st, narrow, medium);
-  } else if (k % kTileK == 0) {
-    launch_tiles<Epi::kPlain>(a, grid, st, narrow, medium);
   } else {
     linear_staged_k<false, false><<<grid, kGemmThreads, 0, st>>>(a);
   }
@@ -714,12 +864,7 @@ int uocr_rocm_linear_bf16x(void* stream, const uint16_t* x, int64_t m, int64_t k
 
 int64_t uocr_rocm_linear_workspace_floats(int64_t m, int64_t k, int64_t n) {
   if (m <= 1 || n <= 0 || k <= 0) return 0;
-  // enough for either tiling a product of few rows may take
-  int64_t s = splits_for(m, k, n);
-  if (m <= kNarrowRows) {
-    const int64_t sn = splits_for(m, k, n, true);
-    s = sn > s ? sn : s;
-  }
+  const int64_t s = splits_for(m, k, n);
   return s > 1 ? s * m * n : 0;
 }
 

@@ -2,12 +2,12 @@
 // (+ bias[n]) with x and w bf16 and y fp32 through hipBLASLt, the ROCm
 // counterpart of the cuBLAS call inside the reference's cuda::linear
 // (src/backend/cuda/ops.cu:268-287: a bf16 GEMM with fp32 compute, then the
-// bias). The hand-written tile kernels (gemm.hip) keep the products with an
-// activation epilogue into bf16 or a row scatter, fp32 x, and few rows; this
-// path takes the plain products (bias, and an add into y, allowed) of at
-// least kLibraryMinRows rows, where the library's tiles run about 1.6x the
-// hand-written ones (865 against 537 TFLOP/s over a dense decoder layer's
-// four projections at 4096 rows, random bf16 operands).
+// bias). The hand-written kernels (gemm.hip) keep the products with an
+// activation epilogue into bf16 or a row scatter, fp32 x, and few rows or
+// few output tiles; this path takes the plain products (bias, and an add into
+// y, allowed) of at least kLibraryMinRows rows that are large enough for the
+// library's tiles to be ahead (4096 x 13696 x 1280: 156 us here, 200 by the
+// hand-written 256 x 128 tiles).
 //
 // In hipBLASLt's column-major terms y^T [n, m] = w [k, n]^T . x^T [k, m]:
 // A = w transposed (lda k), B = x (ldb k), D = y (ldd n), and the bias

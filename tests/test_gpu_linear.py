@@ -290,3 +290,48 @@ def test_library_linear_against_the_tiles(backend, m, k, n, with_bias, request):
     y_tiles = torch.full((m, n), float("nan"), device="cuda")
     backend.linear(xb, wd, y_tiles, bd)
     assert_f32_close(host_f32(y_tiles), host_f32(y), 1e-5, "tiles and library agree")
+
+
+@pytest.mark.parametrize("m,k,n", [
+    (2, 64, 5), (33, 320, 35), (63, 64 * 27, 31), (512, 768, 512),  # 32 x 32 split (and one chain): ragged, 16 x 16 tiles
+    (257, 1024, 1024), (127, 704, 4100), (65, 320, 4099),  # 64 x 32 split, a row past a tile, n off the quads
+    (257, 1024, 3072), (961, 384, 1023),  # 64 x 64 split
+    (900, 896, 1280), (2050, 320, 511), (3000, 64, 260),  # 64 x 64 shared, one step
+    (4097, 320, 1600), (4100, 128, 1666),  # 256 x 128 shared, two steps of 64
+    (3, 2 ** 23, 5)])  # rows of 2^23 columns
+def test_linear_tile_forms(backend, tiles_only, m, k, n):
+    """Every form of the tile kernels at its edges, plain, added into y,
+    scattered and through the activation, against 64-bit sums. Bound: the
+    products are exact in fp32 and every output is a chain (or four) of k / 16
+    matrix-core sums of 16: at most k / 16 + 16 fp32 roundings of partial
+    sums no larger than sum |x| |w|; the fused epilogues bitwise the separate
+    passes."""
+    g = torch.Generator().manual_seed(m + k + n)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16)
+    w = (0.05 * torch.randn(n, k, generator=g)).to(torch.bfloat16)
+    bias = torch.randn(n, generator=g)
+    xd, wd, bd = x.cuda(), w.cuda(), bias.cuda()
+    want = x.double() @ w.double().t() + bias.double()
+    bound = (k / 16 + 16) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t() + bias.double().abs()) + 1e-30
+    y = torch.full((m, n), float("nan"), device="cuda")
+    backend.linear(xd, wd, y, bd)
+    err = (y.double().cpu() - want).abs()
+    assert bool((err <= bound).all()), f"{(err / bound).max():.3g} of the bound"
+    resid = torch.randn(m, n, generator=g).cuda()
+    want_add = resid.clone()
+    backend.add_inplace(want_add, y)
+    got = resid.clone()
+    backend.linear_add(xd, wd, got, torch.empty(1, device="cuda"), bd)
+    assert torch.equal(got, want_add)
+    rows = torch.randperm(m, generator=g)
+    rows[0] = m  # dropped
+    got = resid.clone()
+    backend.linear_add_rows(xd, wd, got, rows.cuda(), bd)
+    want_rows = resid.clone()
+    kept = (rows < m).nonzero().flatten().cuda()
+    want_rows[rows.cuda()[kept]] += y[kept]
+    assert torch.equal(got, want_rows)
+    act, want_act = (torch.empty(m, n, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    backend.linear_act(xd, wd, act, bd)
+    backend.act_to_bf16(y, want_act)
+    assert torch.equal(act, want_act)
