@@ -297,8 +297,13 @@ def _torch():
 
 
 def current_stream() -> int:
-    """torch's current stream on the current device, as the C ABI takes it."""
-    return _torch().cuda.current_stream().cuda_stream
+    """torch's current stream on the current device, as the C ABI takes it.
+
+    Read as the handle itself: torch.cuda.current_stream() builds a Stream
+    object around it, 3.1 us of the 7 that a call of a small op takes on the
+    host (0.2 this way)."""
+    torch = _torch()
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _ptr(t) -> Optional[int]:
