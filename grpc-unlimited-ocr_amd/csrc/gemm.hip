@@ -687,17 +687,17 @@ __global__ __launch_bounds__(kBlock) void round_bf16_k(const float* __restrict__
 
 // The forms of linear_pipe_k. Split forms: four waves over k, a tile to each
 // CU; shared forms: waves over the tile.
-enum class Form { kSplit32, kSplit64x32, kSplit64, kShared64, kShared256, kFar };
+enum class Form { kSplit32, kSplit64x32, kSplit64, kShared64, kShared128, kFar };
 
 // Workgroups the split forms want at most: one a CU. A CU holds one of their
 // workgroups (96 to 147 KB of tiles), so one more tile than this costs a
 // second pass over the chip.
 constexpr int64_t kChipTiles = 256;
-// From this many 64 x 64 tiles the 256 x 128 ones (an eighth of the tiles,
-// half the L2 reads a product) are ahead: 4096 x 2304 x 768 (2304) 34.6
-// against 32.3 us, 2500 x 3072 x 768 (1920) 27.2 against 26.0, 4900 x 768 x
-// 768 (924) and below the other way round.
-constexpr int64_t kShared256Tiles = 1536;
+// Past this many 64 x 64 tiles (three a CU, what it holds at once) the 128 x
+// 128 ones by eight waves are ahead: 4900 x 768 x 768 (924) 25.4 against 16.7
+// us, 3136 x 2304 x 768 (1764) 29 against 20.8, 4096 x 2304 x 768 (2304) 34.6
+// against 33.8; 4096 x 768 x 3072 (768) 40.2 against 44.9.
+constexpr int64_t kSharedTiles = 3 * kChipTiles;
 // Rows of this many columns or more: 256 of them are 2^32 bytes.
 constexpr int64_t kFarColumns = int64_t{1} << 23;
 
@@ -714,15 +714,15 @@ constexpr int64_t kChain = 256;
 
 Form form_of(int64_t m, int64_t n, int64_t k) {
   if (k >= kFarColumns) return Form::kFar;
-  if (k <= kChain) return tiles_of(m, n, 64, 64) < kShared256Tiles ? Form::kShared64 : Form::kShared256;
+  if (k <= kChain) return tiles_of(m, n, 64, 64) <= kSharedTiles ? Form::kShared64 : Form::kShared128;
   if (tiles_of(m, n, 32, 32) <= kChipTiles) return Form::kSplit32;
   if (tiles_of(m, n, 64, 32) <= kChipTiles) return Form::kSplit64x32;
   if (tiles_of(m, n, 64, 64) <= kChipTiles) return Form::kSplit64;
-  return tiles_of(m, n, 64, 64) < kShared256Tiles ? Form::kShared64 : Form::kShared256;
+  return tiles_of(m, n, 64, 64) <= kSharedTiles ? Form::kShared64 : Form::kShared128;
 }
 
 // The runs of k a form sums apart.
-int runs_of(Form form) { return form == Form::kShared64 || form == Form::kShared256 ? 1 : 4; }
+int runs_of(Form form) { return form == Form::kShared64 || form == Form::kShared128 ? 1 : 4; }
 
 // Where the library's larger tiles are the faster ones (us, here / library):
 // past the split forms with a long k (1600 x 768 x 3072, 300 tiles 23.4 /
@@ -754,7 +754,7 @@ void launch_pipe(LinearArgs& a, Form form, hipStream_t st) {
     case Form::kSplit64x32: launch.template operator()<64, 32, 1, 1, 4, 64, 3, false>(); break;
     case Form::kSplit64: launch.template operator()<64, 64, 1, 1, 4, 64, 2, false>(); break;
     case Form::kShared64: launch.template operator()<64, 64, 2, 2, 1, 64, 3, false>(); break;
-    case Form::kShared256: launch.template operator()<256, 128, 4, 2, 1, 32, 3, false>(); break;
+    case Form::kShared128: launch.template operator()<128, 128, 2, 4, 1, 64, 2, false>(); break;
     case Form::kFar: launch.template operator()<32, 32, 1, 1, 4, 64, 3, true>(); break;
   }
 }

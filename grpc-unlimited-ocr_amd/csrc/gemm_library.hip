@@ -6,8 +6,8 @@
 // activation epilogue into bf16 or a row scatter, fp32 x, and few rows or
 // few output tiles; this path takes the plain products (bias, and an add into
 // y, allowed) of at least kLibraryMinRows rows that are large enough for the
-// library's tiles to be ahead (4096 x 13696 x 1280: 156 us here, 200 by the
-// hand-written 256 x 128 tiles).
+// library's tiles to be ahead (4096 x 13696 x 1280: 156 us here, 230 by the
+// hand-written 128 x 128 tiles).
 //
 // In hipBLASLt's column-major terms y^T [n, m] = w [k, n]^T . x^T [k, m]:
 // A = w transposed (lda k), B = x (ldb k), D = y (ldd n), and the bias

@@ -297,7 +297,7 @@ def test_library_linear_against_the_tiles(backend, m, k, n, with_bias, request):
     (257, 1024, 1024), (127, 704, 4100), (65, 320, 4099),  # 64 x 32 split, a row past a tile, n off the quads
     (257, 1024, 3072), (961, 384, 1023),  # 64 x 64 split
     (900, 896, 1280), (2050, 320, 511), (3000, 64, 260),  # 64 x 64 shared, one step
-    (4097, 320, 1600), (4100, 128, 1666),  # 256 x 128 shared, two steps of 64
+    (4097, 320, 1600), (4100, 128, 1666), (2049, 64, 2050),  # 128 x 128 shared, one step, two
     (3, 2 ** 23, 5)])  # rows of 2^23 columns
 def test_linear_tile_forms(backend, tiles_only, m, k, n):
     """Every form of the tile kernels at its edges, plain, added into y,
