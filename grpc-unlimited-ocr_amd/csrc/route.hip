@@ -381,6 +381,49 @@ __device__ __forceinline__ void route_candidates(const PageRanges& r, int nblk, 
   route_candidates_end(nblk, last_remote, cand, slots);
 }
 
+// What a wave selects for one query row: lane j < m comes with the j-th
+// largest key (`mine`); the lanes below k whose block is a candidate are
+// valid, with the block's bias.
+struct Selection {
+  int blk;
+  bool valid;
+  float bias;
+  uint64_t vmask;  // the valid lanes
+  int count;
+};
+
+__device__ __forceinline__ Selection entmax_select(uint64_t mine, int m, int k, const RouteArgs& p, int lane,
+                                                   const unsigned char* cand) {
+#pragma clang fp contract(off)
+  // lane j < m holds the j-th selection
+  const bool have = lane < m;
+  const int blk = have ? key_block(mine) : 0;
+  const float val = have ? key_value(mine) : 0.0f;
+  const float peak = readlane_f32(val, 0);
+  const float v = have ? (val - peak) / 2.0f : 0.0f;
+  // running sums in lane order over the first m lanes (the later lanes'
+  // sums are never read)
+  auto prefix = [m](float x) { return m <= 16 ? prefix_in_order<15>(x) : prefix_in_order<kMaxTop - 1>(x); };
+  const float sum = prefix(v), sum_sq = prefix(v * v);
+  const float rho = static_cast<float>(lane + 1);
+  const float mean = sum / rho, mean_sq = sum_sq / rho;
+  const float ss = rho * (mean_sq - mean * mean);
+  const float delta = fmaxf((1.0f - ss) / rho, 0.0f);
+  const float tau = mean - sqrtf(delta);
+  const int support = __popcll(__ballot(have && tau <= v));
+  const float tau_star = readlane_f32(tau, (support > 1 ? support : 1) - 1);
+  const float t = fmaxf(v - tau_star, 0.0f);
+  const float prob = t * t;
+  const bool valid = lane < k && cand[blk] != 0;
+  const float logp = logf(fmaxf(prob, p.floor));
+  const float logp_sum = readlane_f32(prefix(valid ? logp : 0.0f), k - 1);
+  const uint64_t vmask = __ballot(valid);
+  const int count = __popcll(vmask);
+  const float mu = logp_sum / static_cast<float>(count > 1 ? count : 1);
+  const float bias = (logp - mu) / p.sigma;
+  return {blk, valid, bias, vmask, count};
+}
+
 // The selection and the key mask of one query at position pos over nblk
 // blocks (z[b], raw scores of the blocks b <= last_remote; other entries are
 // not read), given cand: x = clamp(z) * idx_scale on candidates and -1e4
@@ -474,32 +517,11 @@ __device__ void route_select(const float* z, int nblk, int64_t pos, int64_t keys
     }
   }
   if (wave == 0) {
-    // lane j < m holds the j-th selection
-    const bool have = lane < m;
-    const int blk = have ? key_block(mine) : 0;
-    const float val = have ? key_value(mine) : 0.0f;
-    const float peak = readlane_f32(val, 0);
-    const float v = have ? (val - peak) / 2.0f : 0.0f;
-    // running sums in lane order over the first m lanes (the later lanes'
-    // sums are never read)
-    auto prefix = [m](float x) { return m <= 16 ? prefix_in_order<15>(x) : prefix_in_order<kMaxTop - 1>(x); };
-    const float sum = prefix(v), sum_sq = prefix(v * v);
-    const float rho = static_cast<float>(lane + 1);
-    const float mean = sum / rho, mean_sq = sum_sq / rho;
-    const float ss = rho * (mean_sq - mean * mean);
-    const float delta = fmaxf((1.0f - ss) / rho, 0.0f);
-    const float tau = mean - sqrtf(delta);
-    const int support = __popcll(__ballot(have && tau <= v));
-    const float tau_star = readlane_f32(tau, (support > 1 ? support : 1) - 1);
-    const float t = fmaxf(v - tau_star, 0.0f);
-    const float prob = t * t;
-    const bool valid = lane < k && sh.cand[blk] != 0;
-    const float logp = logf(fmaxf(prob, p.floor));
-    const float logp_sum = readlane_f32(prefix(valid ? logp : 0.0f), k - 1);
-    const uint64_t vmask = __ballot(valid);
-    const int count = __popcll(vmask);
-    const float mu = logp_sum / static_cast<float>(count > 1 ? count : 1);
-    const float bias = (logp - mu) / p.sigma;
+    const Selection sel = entmax_select(mine, m, k, p, lane, sh.cand);
+    const int blk = sel.blk, count = sel.count;
+    const bool valid = sel.valid;
+    const float bias = sel.bias;
+    const uint64_t vmask = sel.vmask;
     if (valid) sh.block_bias[blk] = bias;
     if (segs != nullptr) {
       const int64_t wkeys = static_cast<int64_t>(p.local_blocks) * p.block_size;
@@ -685,6 +707,95 @@ __global__ __launch_bounds__(kRouteBlock) void route_rows_k(const float* __restr
   const int64_t page = query_page != nullptr ? query_page[row] : one_page;
   route_row(z + row * nblk, nblk, first_pos + row, keys, page, block_min, block_max, prompt_blocks, p, sh.lds(),
             mask + row * keys);
+}
+
+// Prompt rows of at most kWaveRouteBlocks blocks: a wave a row, four blocks a
+// lane, no barrier. A workgroup of 16 waves a row spends its time between
+// barriers and in the one wave that forms the entmax (4096 rows of 128
+// blocks 50 us); a row's instructions are few enough for one wave, and 16 rows
+// on a CU hide each other's latencies behind the mask's stores, which bound
+// this form (64 MB at 4096 x 4096). The same keys, the same entmax: bitwise
+// route_rows_k.
+constexpr int kWaveRouteBlocks = 4 * kWave;
+constexpr int kRowWaves = 4;
+
+__global__ __launch_bounds__(kRowWaves* kWave) void route_rows_wave_k(
+    const float* __restrict__ z, int64_t rows, int nblk, int64_t first_pos, int64_t keys,
+    const int64_t* __restrict__ block_min, const int64_t* __restrict__ block_max, int64_t prompt_blocks,
+    const int64_t* __restrict__ query_page, int64_t one_page, RouteArgs p, float* __restrict__ mask) {
+  __shared__ float biases[kRowWaves][kWaveRouteBlocks];
+  __shared__ unsigned char cands[kRowWaves][kWaveRouteBlocks];
+  const int lane = threadIdx.x & (kWave - 1), wave = wave_in_block();
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * kRowWaves + wave;
+  if (row >= rows) return;
+  float* const block_bias = biases[wave];
+  unsigned char* const cand = cands[wave];
+  const int64_t page = query_page != nullptr ? query_page[row] : one_page;
+  const int64_t pos = first_pos + row;
+  const int64_t last_remote = pos / p.block_size - p.local_blocks;
+  const float* const zr = z + row * nblk;
+  float zv[4];
+  bool allowed[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int b = lane + kWave * i;
+    zv[i] = b < nblk ? zr[b] : 0.0f;
+    int64_t lo = -1, hi = -1;
+    if (page >= 0 && b < nblk && b < prompt_blocks) {
+      lo = block_min[b];
+      hi = block_max[b];
+    }
+    allowed[i] = b < nblk && b <= last_remote && page >= 0 && lo >= 0 && lo <= page && page <= hi;
+  }
+  const bool none = __ballot(allowed[0] || allowed[1] || allowed[2] || allowed[3]) == 0;
+  uint64_t key[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int b = lane + kWave * i;
+    const bool c = none ? b <= last_remote : allowed[i];
+    key[i] = b < nblk ? order_key(c ? clamp_act(zv[i]) * p.idx_scale : kEntmaxMasked, b) : 0;
+    cand[b] = c;
+    block_bias[b] = -INFINITY;
+  }
+  const int m = p.top_m < nblk ? (p.top_m > 1 ? p.top_m : 1) : (nblk > 1 ? nblk : 1);
+  const int k = p.top_k < m ? (p.top_k > 1 ? p.top_k : 1) : m;
+  const uint64_t mine = wave_top<4>(key, m, lane);
+  // the wave's own LDS writes, read by its other lanes from here on
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  const Selection sel = entmax_select(mine, m, k, p, lane, cand);
+  if (sel.valid) block_bias[sel.blk] = sel.bias;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+
+  // key j < end: 0 from `near` on, its block's bias before; -inf from end on
+  const int64_t window = static_cast<int64_t>(p.local_blocks) * p.block_size;
+  const int64_t end = pos + 1 < keys ? pos + 1 : keys;
+  const int64_t near = pos + 1 - window > 0 ? pos + 1 - window : 0;
+  const uint32_t bs = static_cast<uint32_t>(p.block_size);
+  float* const out = mask + row * keys;
+  auto value = [&](int64_t j) {
+    return j >= end ? -INFINITY : j >= near ? 0.0f : block_bias[static_cast<uint32_t>(j) / bs];
+  };
+  int64_t j0 = 0;
+  if ((reinterpret_cast<uintptr_t>(out) & 15u) == 0) {  // 16-byte stores
+    const int64_t quads = keys / 4;
+    for (int64_t c = lane; c < quads; c += kWave) {
+      const int64_t j = 4 * c;
+      float v[4];
+      if (bs % 4 == 0) {  // a quad's keys share their block
+        const float bias = j < end && j < near ? block_bias[static_cast<uint32_t>(j) / bs] : 0.0f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = j + e >= end ? -INFINITY : j + e >= near ? 0.0f : bias;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = value(j + e);
+      }
+      *reinterpret_cast<float4*>(out + j) = make_float4(v[0], v[1], v[2], v[3]);
+    }
+    j0 = 4 * quads;
+  }
+  for (int64_t j = j0 + lane; j < keys; j += kWave) out[j] = value(j);
 }
 
 // One decode query, lengths from the StepState: mask [pos + 1].
@@ -971,6 +1082,12 @@ int uocr_rocm_route_blocks(void* stream, const float* z, int64_t rows, int64_t n
                kWhat, "prompt blocks without their pages");
   UOCR_REQUIRE(z != nullptr && mask != nullptr, kWhat, "null pointer");
   clear_launch_error();
+  if (nblk <= kWaveRouteBlocks) {
+    route_rows_wave_k<<<static_cast<unsigned>((rows + kRowWaves - 1) / kRowWaves), kRowWaves * kWave, 0,
+                        as_stream(stream)>>>(z, rows, static_cast<int>(nblk), first_pos, keys, block_min, block_max,
+                                             prompt_blocks, query_page, one_page, p, mask);
+    return check_launch(kWhat);
+  }
   route_rows_k<<<static_cast<unsigned>(rows), kRouteBlock, 0, as_stream(stream)>>>(
       z, static_cast<int>(nblk), first_pos, keys, block_min, block_max, prompt_blocks, query_page, one_page, p, mask);
   return check_launch(kWhat);

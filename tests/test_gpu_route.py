@@ -322,3 +322,35 @@ def test_route_rejects_bad_shapes(backend):
     with pytest.raises(ValueError, match="block_size must be in"):
         backend.block_summaries(torch.zeros(10, 8, device="cuda"), torch.zeros(8, device="cuda"), 65,
                                 torch.zeros(8, device="cuda"))
+
+
+@pytest.mark.parametrize("nblk,bs,first,rows,past", [
+    (1, 32, 0, 20, 0), (5, 32, 3, 150, 0), (63, 16, 900, 7, 3), (64, 32, 2001, 40, 1), (65, 20, 1200, 70, 0),
+    (128, 32, 4000, 90, 6), (255, 3, 700, 60, 2), (256, 64, 16300, 70, 5), (257, 32, 8100, 9, 0)])
+def test_route_blocks_is_route_step_row_by_row(backend, nblk, bs, first, rows, past):
+    """A prompt's rows (a wave a row up to 256 blocks, a workgroup a row past
+    them) against the one-query step at each row's position, bitwise: tied
+    scores, NaN in blocks no row may read, pages without a remote block,
+    block sizes off four and off powers of two, keys past the last position
+    and rows of keys off 16 bytes."""
+    g = np.random.default_rng(nblk)
+    p = backend.RouteParams(block_size=bs)
+    keys = first + rows + past
+    z = normal(370 + nblk, (rows, nblk), 3.0)
+    z[:, : nblk // 2 : 3] = 0.25
+    for r in range(rows):
+        z[r, max(0, (first + r) // bs - 3):] = np.nan
+    lo = g.integers(-1, 4, nblk)
+    hi = lo + g.integers(0, 2, nblk)
+    qp = g.integers(-1, 7, rows)
+    mask = torch.full((rows, keys), float("nan"), device="cuda")
+    lo_d, hi_d, zd = dev_i64(lo.astype(np.int64)), dev_i64(hi.astype(np.int64)), dev_f32(z)
+    backend.route_blocks(zd, first, keys, lo_d, hi_d, dev_i64(qp.astype(np.int64)), -1, p, mask)
+    got = host_f32(mask)
+    for r in range(rows):
+        pos = first + r
+        one = torch.full((pos + 1,), float("nan"), device="cuda")
+        backend.route_step(zd[r].contiguous(), lo_d, hi_d, state_of(pos, tok=pos, page=0, query_page=int(qp[r])), p, one)
+        want = host_f32(one)
+        assert np.array_equal(got[r, : pos + 1].view(np.uint32), want.view(np.uint32)), f"row {r}"
+        assert np.all(np.isneginf(got[r, pos + 1:]))
