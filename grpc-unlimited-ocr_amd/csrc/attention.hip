@@ -29,10 +29,8 @@
 // consecutive products are one 16-byte read; each 32 columns of the head are
 // 16 products into 16 accumulators.
 //
-// With a mask, a wave reads its 32 x 32 block of the mask before a tile's
-// products and skips the tile where every entry is -inf: a causal mask's
-// upper tiles, and all but the selected blocks (32 keys each) of the
-// decoder's routed mask, cost only their share of the K/V staging.
+// With a mask the 4 waves of a workgroup take the same 32 query rows and the
+// live key tiles of those in turn (attention_mask_k).
 //
 // Arithmetic: fp32 products and sums on the matrix cores; the scores are
 // scaled, then the bias added (the reference's order); e = exp(s - running
@@ -57,7 +55,7 @@ constexpr float kLog2e = 1.4426950408889634f;
 // kRelPosTable: kRelPosRows with the per-query dot products read from the
 // table rel_dots_k formed in memory rather than copied into LDS (4 waves a
 // workgroup: no LDS for them).
-enum class Bias { kNone, kMask, kRelPos, kRelPosRows, kRelPosTable };
+enum class Bias { kNone, kRelPos, kRelPosRows, kRelPosTable };
 template <Bias kBias>
 constexpr bool rel_pos() {
   return kBias == Bias::kRelPos || kBias == Bias::kRelPosRows || kBias == Bias::kRelPosTable;
@@ -87,7 +85,7 @@ struct AttnArgs {
   int64_t ldq, sq, ldk, sk, ldv, sv, ldo, so;  // row and slice strides (elements)
   int rows, keys;
   float scale;
-  const float* mask;  // [rows, mask_ld] (kMask)
+  const float* mask;  // [rows, mask_ld] (attention_mask_k and the split-operand form)
   int64_t mask_ld;
   const float* rh;  // [h, h, hd] (kRelPos, kRelPosRows)
   const float* rw;  // [w, w, hd]
@@ -112,12 +110,12 @@ struct AttnArgs {
   // dot-table launch (kv_tiles_of), for key tiles of x3_rows grid rows
   uint16_t* kvx = nullptr;
   int x3_rows = -1;
-  // non-null (attention_k with a mask): the mask's live-tile map (a bit per
-  // 128 query rows and 32-key tile, map_words words per row block); a row
-  // block's walk is cut into `runs` runs of run_tiles live tiles, and where
-  // a block takes more than one, each run leaves per row (m, l) in part_ml
-  // and its unnormalised output in part_o ([slices][row blocks][runs][128
-  // rows]) for the merge launch
+  // attention_mask_k, non-null: the mask's live-tile map (a bit per 128 query
+  // rows and 32-key tile, map_words words per row block); a row block's walk
+  // is cut into `runs` runs of run_tiles live tiles, and where a block takes
+  // more than one, each run leaves per row (m, l) in part_ml and its
+  // unnormalised output in part_o ([slices][row blocks][runs][128 rows]) for
+  // the merge launch
   const uint32_t* map = nullptr;
   int map_words = 0, run_tiles = 0, runs = 1;
   float* part_o = nullptr;
@@ -261,11 +259,7 @@ __global__ __launch_bounds__(64 * waves_of<kBias>()) void attention_k(const Attn
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int hl = lane >> 5, c = lane & 31;
   const int64_t slice = blockIdx.y;
-  // with a mask, the last row blocks first (under a causal mask the longest
-  // walks); with a map, workgroup x is (row block, run)
-  const int run = kBias == Bias::kMask ? static_cast<int>(blockIdx.x) % a.runs : 0;
-  const int rblk = kBias == Bias::kMask ? static_cast<int>(gridDim.x / a.runs - 1 - blockIdx.x / a.runs)
-                                        : static_cast<int>(blockIdx.x);
+  const int rblk = static_cast<int>(blockIdx.x);
   const int q0 = rblk * kQueriesPerBlock + wave * kQueriesPerWave;
   const int qrow = q0 + c;
   const bool qin = qrow < a.rows;
@@ -273,36 +267,12 @@ __global__ __launch_bounds__(64 * waves_of<kBias>()) void attention_k(const Attn
   const float* kb = a.k + slice_at(a, slice, a.sk, a.ik);
   const float* vb = a.v + slice_at(a, slice, a.sv, a.iv);
 
-  // the tiles this workgroup walks: every one, or with a map the live tiles
-  // of its run (uniform: scalar reads)
   const int tiles = (a.keys + kKeyTile - 1) / kKeyTile;
-  const bool mapped = kBias == Bias::kMask && a.map != nullptr;
-  const uint32_t* tmap = mapped ? a.map + static_cast<int64_t>(rblk) * a.map_words : nullptr;
-  MapCursor cursor{tmap, -1, 0u};
   const int64_t orow = slice_at(a, slice, a.so, a.io) + static_cast<int64_t>(qrow) * a.ldo;
-  int first = 0, block_runs = 1;
-  if (mapped) {
-    const int live = live_tiles(tmap, a.map_words);
-    block_runs = (live + a.run_tiles - 1) / a.run_tiles;
-    if (live == 0) {  // no key attended by any row of the block: zeros
-      if (run == 0 && qin) {
-#pragma unroll
-        for (int e = 0; e < HD / 8; ++e) store4(a, orow + 8 * e + 4 * hl, 0.0f, 0.0f, 0.0f, 0.0f);
-      }
-      return;
-    }
-    if (run >= block_runs) return;  // uniform, before any barrier
-    first = -1;
-    for (int skip = run * a.run_tiles; skip >= 0; --skip) first = next_live_tile(cursor, tiles, first);
-  }
-  // the tile after t (i: t's place in the run), or tiles
-  auto after = [&](int t, int i) {
-    return mapped ? (i + 1 < a.run_tiles ? next_live_tile(cursor, tiles, t) : tiles) : t + 1;
-  };
 
   // the first tile's loads go out first
   float4 kr[T::kPerThread], vr[T::kPerThread];
-  load_tile<HD, kThreads>(a, kb, vb, first * kKeyTile, kr, vr);
+  load_tile<HD, kThreads>(a, kb, vb, 0, kr, vr);
 
   // this lane's half of its query row
   float qv[kHalf];
@@ -366,9 +336,8 @@ __global__ __launch_bounds__(64 * waves_of<kBias>()) void attention_k(const Attn
   }
 
   store_tile<HD, kThreads>(ks, vs, kr, vr);
-  int nxt = after(first, 0);  // the tile after the current one
   if constexpr (kStages == 2) {
-    if (nxt < tiles) load_tile<HD, kThreads>(a, kb, vb, nxt * kKeyTile, kr, vr);
+    if (1 < tiles) load_tile<HD, kThreads>(a, kb, vb, kKeyTile, kr, vr);
   }
   __syncthreads();
 
@@ -379,61 +348,22 @@ __global__ __launch_bounds__(64 * waves_of<kBias>()) void attention_k(const Attn
     for (int r = 0; r < 16; ++r) o[b][r] = 0.0f;
   }
   float m = -INFINITY, l = 0.0f;
-  // With a mask, this wave's 32 x 32 block of it (register r: key 8 (r / 4)
-  // + 4 h + r % 4 of the tile; -inf past the keys or the rows), read a tile
-  // ahead: where every entry is -inf (a causal or routed mask's dead tiles)
-  // the wave skips the tile's products and softmax; the tile's K and V
-  // still reach LDS for the other waves.
-  constexpr int kMk = kBias == Bias::kMask ? 16 : 1;
-  float mk[kMk], mn[kMk];
-  const bool vec = kBias == Bias::kMask && mask_vec(a.mask, a.mask_ld);
-  const float* mrow = a.mask + static_cast<int64_t>(qin ? qrow : 0) * a.mask_ld;
-  auto load_mask = [&](int tt, float (&dst)[kMk]) {
-    if constexpr (kBias == Bias::kMask) {
-      const bool whole = vec && (tt + 1) * kKeyTile <= a.keys;  // uniform
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int key4 = tt * kKeyTile + 8 * g + 4 * hl;
-        float4 v = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
-        if (whole) {
-          if (qin) v = *reinterpret_cast<const float4*>(mrow + key4);
-        } else if (qin && key4 < a.keys) {
-          v = mask4(mrow, key4, a.keys, vec);
-        }
-        dst[4 * g] = v.x;
-        dst[4 * g + 1] = v.y;
-        dst[4 * g + 2] = v.z;
-        dst[4 * g + 3] = v.w;
-      }
-    }
-  };
-  load_mask(first, mk);
   int st = 0;  // the LDS stage holding the current tile
-  for (int t = first, i = 0; t < tiles; ++i) {
+  for (int t = 0; t < tiles; ++t) {
     const int key0 = t * kKeyTile;
-    const bool more = nxt < tiles;
-    int nxt2 = tiles;  // (two stages) the tile after nxt, requested now
+    const bool more = t + 1 < tiles;
     if constexpr (kStages == 2) {
       if (more) store_tile<HD, kThreads>(ks + (st ^ 1) * kKElems, vs + (st ^ 1) * kVElems, kr, vr);
-      nxt2 = more ? after(nxt, i + 1) : tiles;
-      if (nxt2 < tiles) load_tile<HD, kThreads>(a, kb, vb, nxt2 * kKeyTile, kr, vr);
+      if (t + 2 < tiles) load_tile<HD, kThreads>(a, kb, vb, (t + 2) * kKeyTile, kr, vr);  // requested now
     } else {
-      if (more) load_tile<HD, kThreads>(a, kb, vb, nxt * kKeyTile, kr, vr);
+      if (more) load_tile<HD, kThreads>(a, kb, vb, (t + 1) * kKeyTile, kr, vr);
     }
-    load_mask(more ? nxt : t, mn);
     const float* kcur = ks + st * kKElems;
     const float* vcur = vs + st * kVElems;
 
     // A wave whose rows all lie past the last query row (the tail workgroup
     // of a slice) only helps stage the tiles.
-    bool live = q0 < a.rows;
-    if constexpr (kBias == Bias::kMask) {
-      bool any = false;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) any = any || mk[r] != -INFINITY;
-      live = live && __ballot(any) != 0;
-    }
-    if (live) {
+    if (q0 < a.rows) {
       // S^T = K Q^T: 32 keys x 32 queries
       f32x16 s;
 #pragma unroll
@@ -494,9 +424,7 @@ __global__ __launch_bounds__(64 * waves_of<kBias>()) void attention_k(const Attn
       for (int r = 0; r < 16; ++r) {
         const int off = 8 * (r / 4) + 4 * hl + (r % 4), key = key0 + off;
         float x = s[r] * a.scale;
-        if constexpr (kBias == Bias::kMask) {
-          x = x + mk[r];
-        } else if constexpr (kBias == Bias::kRelPos) {
+        if constexpr (kBias == Bias::kRelPos) {
           int ky = gky[r / 4], kx = gkx[r / 4] + r % 4;
           while (kx >= a.w) {  // at most once for a grid 4 or more wide
             kx -= a.w;
@@ -557,36 +485,10 @@ __global__ __launch_bounds__(64 * waves_of<kBias>()) void attention_k(const Attn
         __syncthreads();
       }
     }
-    if constexpr (kBias == Bias::kMask) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) mk[r] = mn[r];
-    }
-    t = nxt;
-    if constexpr (kStages == 2) {
-      nxt = nxt2;
-      st ^= 1;
-    } else {
-      nxt = more ? after(t, i + 1) : tiles;
-    }
+    if constexpr (kStages == 2) st ^= 1;
   }
 
   if (!qin) return;
-  if (mapped && block_runs > 1) {
-    // the run's partial record: (m, l) (lane half 0) and O unnormalised
-    const int row_blocks = static_cast<int>(gridDim.x) / a.runs;
-    const int64_t rec = ((slice * row_blocks + rblk) * a.runs + run) * kQueriesPerBlock + (qrow - rblk * kQueriesPerBlock);
-    if (hl == 0) *reinterpret_cast<float2*>(a.part_ml + 2 * rec) = make_float2(m, l);
-#pragma unroll
-    for (int b = 0; b < kDBlocks; ++b) {
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int d = 32 * b + 8 * g + 4 * hl;
-        *reinterpret_cast<float4*>(a.part_o + rec * HD + d) =
-            make_float4(o[b][4 * g], o[b][4 * g + 1], o[b][4 * g + 2], o[b][4 * g + 3]);
-      }
-    }
-    return;
-  }
   const float inv = l > 0.0f ? 1.0f / l : 0.0f;
 #pragma unroll
   for (int b = 0; b < kDBlocks; ++b) {
@@ -1605,6 +1507,416 @@ __global__ __launch_bounds__(64 * kSplitWaves) void attention_keysplit_k(const A
   store4(a, op + 4, acc[4] * inv, acc[5] * inv, acc[6] * inv, acc[7] * inv);
 }
 
+// ---- a mask: 32 query rows a workgroup, their live tiles over its waves ---------
+//
+// A mask leaves each 32 query rows few of the key tiles (the decoder's routed
+// mask about a quarter), and other rows other tiles: with 128 rows a
+// workgroup, as without a mask, the waves wait for each other at every tile
+// that any of them reads. Here the 4 waves of a workgroup take the same 32
+// query rows. They first scan the rows' mask (256 keys a wave at a time, all
+// 32 rows in flight) into a bit a tile, and wave w then walks the live tiles
+// w, w + 4, ...: no barrier, K, V and mask tiles of its own. A tile's products
+// take 8192 clocks of the matrix cores at head dim 128 and 32 KB of K and V,
+// 16 bytes a clock for the CU's four waves, which L2 gives without sharing.
+// The tiles come straight from memory into the wave's LDS (a lane reading its
+// operands from memory takes a cache line a lane, 64 clocks a read, and was
+// bound by that): the next tile's K and mask under the softmax and the
+// values' product, its V under the next scores' product. At the end the
+// waves' records (max, total, values) are combined through LDS in wave order.
+// The products, the online softmax and the roundings are attention_k's.
+//
+// With a workspace the map of 128 rows a bit (mask_tiles_k) names the spans
+// worth scanning, or, where the row groups leave CUs idle, cuts a block's walk
+// into runs, whose records x3m_merge_k combines.
+//
+// us, 128 rows a workgroup before / now (10 heads x 4096 x 128): routed 720 /
+// 384, causal 1231 / 687; 12 x 300 x 64 over 1000 keys causal 122 / 45. A live
+// tile takes a wave 13000 clocks at head dim 128, the matrix cores 8192 of
+// them; one workgroup holds a CU's LDS, so its scan (5 TB/s of mask over the
+// chip) and its first reads stand alone. Half the LDS and two workgroups a CU
+// (K and V in turn in one place) had the accumulators spill and took 498 us
+// routed; K and V read by the lanes that use them, without LDS, 421.
+constexpr int kWalkTiles = 1024;  // tiles a scan covers
+constexpr int kWalkWaves = 4;
+constexpr int kScanRows = 16;
+
+template <int HD>
+__global__ __launch_bounds__(64 * kWalkWaves, 1) void attention_mask_k(const AttnArgs a, int first_group,
+                                                                     int row_groups) {
+  constexpr int kHalf = HD / 2, kDBlocks = HD / 32, kP = HD + 4;
+  constexpr int kTileElems = kKeyTile * HD, kMaskElems = kQueriesPerWave * kKeyTile;
+  constexpr int kStage = 2 * kTileElems + kMaskElems;  // a wave's K, V and mask tiles
+  // 144 KB at head dim 128. The live words take the tiles' place before a walk,
+  // the waves' records after it.
+  __shared__ __attribute__((aligned(16))) float stages[kWalkWaves * kStage];
+  constexpr int kVals = kWalkWaves * kQueriesPerWave * kP;
+  static_assert(kWalkWaves * kStage >= kVals + 2 * kWalkWaves * kQueriesPerWave);
+  uint32_t* const live_words = reinterpret_cast<uint32_t*>(stages);
+  const int lane = threadIdx.x & 63, wave = wave_in_block();
+  const int hl = lane >> 5, c = lane & 31;
+  // slice by slice, the last row groups first (under a causal mask the
+  // longest walks); an XCD's workgroups share their slices' K and V in its L2
+  const unsigned id = xcd_block(blockIdx.x, gridDim.x);
+  const unsigned per = static_cast<unsigned>(row_groups) * static_cast<unsigned>(a.runs);
+  const int64_t slice = id / per;
+  const int at = static_cast<int>(id - slice * per);
+  const int group = first_group + row_groups - 1 - at / a.runs, run = at % a.runs;
+  const int q0 = group * kQueriesPerWave, qrow = q0 + c;
+  const bool qin = qrow < a.rows;
+  const float* qb = a.q + slice_at(a, slice, a.sq, a.iq);
+  const float* kb = a.k + slice_at(a, slice, a.sk, a.ik);
+  const float* vb = a.v + slice_at(a, slice, a.sv, a.iv);
+  const int tiles = (a.keys + kKeyTile - 1) / kKeyTile;
+
+  // the tiles [begin, end) of this run of the row block's map
+  const int rblk = q0 / (4 * kQueriesPerWave);
+  const uint32_t* tmap = a.map != nullptr ? a.map + static_cast<int64_t>(rblk) * a.map_words : nullptr;
+  int begin = 0, end = tiles, block_runs = 1;
+  if (a.runs > 1) {
+    block_runs = (live_tiles(tmap, a.map_words) + a.run_tiles - 1) / a.run_tiles;
+    if (run > 0 && run >= block_runs) return;  // uniform, before any barrier
+    MapCursor cursor{tmap, -1, 0u};
+    begin = -1;
+    for (int skip = run * a.run_tiles; skip >= 0; --skip) begin = next_live_tile(cursor, tiles, begin);
+    end = begin;
+    for (int n = 0; n < a.run_tiles && end < tiles; ++n) end = next_live_tile(cursor, tiles, end);
+  }
+
+  f32x16 o[kDBlocks];
+#pragma unroll
+  for (int b = 0; b < kDBlocks; ++b) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[b][r] = 0.0f;
+  }
+  float m = -INFINITY, l = 0.0f;
+
+  const bool vec = mask_vec(a.mask, a.mask_ld);
+  float* const ks = stages + wave * kStage;
+  float* const vs = ks + kTileElems;
+  float* const ms = vs + kTileElems;
+  const uint32_t ks_lds = lds_address(ks), vs_lds = lds_address(vs), ms_lds = lds_address(ms);
+  // A tile's rows in LDS, 16-byte chunk x of row r at x ^ (r % 16) for K (the
+  // scores' reads of 16 rows then cover the banks), x ^ 8 (r / 4 % 2) for V
+  // (the two lane halves read rows four apart), x ^ (r / 2 % 8) for the
+  // mask. Lane l of a load writes chunk l of its 64; keys past the end read
+  // the last one (their scores are masked, their values set to zero).
+  constexpr int kRowChunks = HD / 4, kRowsALoad = kWave / kRowChunks, kTileLoads = kKeyTile / kRowsALoad;
+  constexpr int kMaskLoads = kQueriesPerWave / 8;
+  // The usual tile, whole and with row strides that fit a lane's 32-bit offset:
+  // one scalar base a load and an offset a lane; else a 64-bit address a lane.
+  const bool near = a.ldk < (1 << 24) && a.ldv < (1 << 24) && a.mask_ld < (1 << 24);
+  const int lrow = lane / kRowChunks, lchunk = lane % kRowChunks;
+  const uint32_t k_off = static_cast<uint32_t>(lrow * a.ldk * 4) + 16 * static_cast<uint32_t>(lchunk ^ lrow);
+  const uint32_t v_off = static_cast<uint32_t>(lrow * a.ldv * 4);
+  auto stage_rows = [&](uint32_t lds, const float* src, int64_t ld, int t, bool is_k) {
+    if (near && (t + 1) * kKeyTile <= a.keys) {  // uniform
+      const char* row = reinterpret_cast<const char*>(src + static_cast<int64_t>(t) * kKeyTile * ld);
+      int64_t step = kRowsALoad * ld * 4;
+      asm volatile("" : "+s"(step));  // added load by load: 16 multiples kept ahead are as many scalar pairs
+#pragma unroll
+      for (int i = 0; i < kTileLoads; ++i) {
+        const int r = kRowsALoad * i;  // its bits and lrow's are apart
+        const uint32_t off = is_k ? k_off ^ (16u * (r & 15)) : v_off + 16 * static_cast<uint32_t>(lchunk ^ (8 * ((r >> 2) & 1)));
+        dma16(lds + i * kWave * 16, row, off);
+        row += step;
+      }
+      return;
+    }
+#pragma unroll 1
+    for (int i = 0; i < kTileLoads; ++i) {
+      const int r = kRowsALoad * i + lrow;
+      const int from = is_k ? lchunk ^ (r & 15) : lchunk ^ (8 * ((r >> 2) & 1));
+      const int key = min(t * kKeyTile + r, a.keys - 1);
+      dma16(lds + i * kWave * 16, reinterpret_cast<const char*>(src),
+            static_cast<uint64_t>((static_cast<int64_t>(key) * ld + 4 * from) * 4));
+    }
+  };
+  uint32_t m_off[kMaskLoads];
+#pragma unroll
+  for (int i = 0; i < kMaskLoads; ++i) {
+    const int r = 8 * i + lane / 8, from = (lane % 8) ^ ((r >> 1) & 7);
+    m_off[i] = static_cast<uint32_t>(min(r, a.rows - 1 - q0) * a.mask_ld * 4) + 16 * from;
+  }
+  const char* const m_base = reinterpret_cast<const char*>(a.mask + static_cast<int64_t>(q0) * a.mask_ld);
+  auto stage_k = [&](int t) {
+    stage_rows(ks_lds, kb, a.ldk, t, true);
+    if (vec && near && (t + 1) * kKeyTile <= a.keys) {  // uniform
+#pragma unroll
+      for (int i = 0; i < kMaskLoads; ++i) {
+        dma16(ms_lds + i * kWave * 16, m_base + static_cast<int64_t>(t) * kKeyTile * 4, m_off[i]);
+      }
+      return;
+    }
+    // lane: row c, keys 16 hl .. + 15
+    const float* mrow = a.mask + static_cast<int64_t>(min(qrow, a.rows - 1)) * a.mask_ld;
+#pragma unroll 1
+    for (int j = 0; j < 4; ++j) {
+      const int key = t * kKeyTile + 16 * hl + 4 * j;
+      float4 x;
+      x.x = mrow[min(key, a.keys - 1)];
+      x.y = mrow[min(key + 1, a.keys - 1)];
+      x.z = mrow[min(key + 2, a.keys - 1)];
+      x.w = mrow[min(key + 3, a.keys - 1)];
+      *reinterpret_cast<float4*>(ms + c * kKeyTile + 4 * ((4 * hl + j) ^ ((c >> 1) & 7))) = x;
+    }
+  };
+  auto stage_v = [&](int t) { stage_rows(vs_lds, vb, a.ldv, t, false); };
+
+  for (int base = begin & ~7; base < end; base += kWalkTiles) {
+    // a bit a tile of [base, base + kWalkTiles): some row's entry not -inf
+    const int span = end - base < kWalkTiles ? end - base : kWalkTiles;
+    __syncthreads();  // the words before are read
+    for (int s = wave; s < kWalkTiles / 8; s += kWalkWaves) {
+      const int t8 = base + 8 * s;
+      uint32_t bits = 0;
+      int64_t ld = a.mask_ld;
+      asm volatile("" : "+s"(ld));  // 32 row offsets formed here, not kept over the kernel in as many scalar pairs
+      if (8 * s < span && (tmap == nullptr || ((tmap[t8 >> 5] >> (t8 & 31)) & 0xffu) != 0)) {
+        // every read in range and unconditional (rows and keys past the end
+        // read the last ones), so that kScanRows rows are in flight at once
+        const int key4 = t8 * kKeyTile + 4 * lane;
+        const int rlast = a.rows - 1 - q0 < kQueriesPerWave ? a.rows - 1 - q0 : kQueriesPerWave - 1;
+        const float* const mp = a.mask + static_cast<int64_t>(q0) * a.mask_ld;
+        bool any = false;
+#pragma unroll
+        for (int half = 0; half < kQueriesPerWave; half += kScanRows) {
+          float4 x[kScanRows];
+          if (vec) {
+            const int at4 = key4 < a.keys ? key4 : (a.keys - 1) & ~3;
+#pragma unroll
+            for (int r = 0; r < kScanRows; ++r) {
+              x[r] = *reinterpret_cast<const float4*>(mp + static_cast<int64_t>(min(half + r, rlast)) * ld + at4);
+            }
+          } else {
+            const int k0 = min(key4, a.keys - 1), k1 = min(key4 + 1, a.keys - 1), k2 = min(key4 + 2, a.keys - 1),
+                      k3 = min(key4 + 3, a.keys - 1);
+#pragma unroll
+            for (int r = 0; r < kScanRows; ++r) {
+              const float* const row = mp + static_cast<int64_t>(min(half + r, rlast)) * ld;
+              x[r] = make_float4(row[k0], row[k1], row[k2], row[k3]);
+            }
+          }
+#pragma unroll
+          for (int r = 0; r < kScanRows; ++r) {
+            // no short circuit: a branch would take the reads behind it
+            any = any | ((x[r].x != -INFINITY) & (key4 < a.keys)) | ((x[r].y != -INFINITY) & (key4 + 1 < a.keys)) |
+                  ((x[r].z != -INFINITY) & (key4 + 2 < a.keys)) | ((x[r].w != -INFINITY) & (key4 + 3 < a.keys));
+          }
+        }
+        const uint64_t v = __ballot(any);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) bits |= ((v >> (8 * j)) & 0xffu) != 0 ? (1u << j) : 0u;
+        if (t8 < begin) bits &= 0xffu << (begin - t8);
+        if (t8 + 8 > end) bits &= (1u << (end - t8)) - 1u;
+      }
+      if (lane == 0) reinterpret_cast<uint8_t*>(live_words)[s] = static_cast<uint8_t>(bits);
+    }
+    __syncthreads();
+    const uint32_t word = live_words[lane & 31];
+    __syncthreads();  // the words are read
+    // this lane's half of its query row, after the scan's registers; a row
+    // past the last computes the last's and is not stored
+    float qv[kHalf];
+    {
+      const float* p = qb + static_cast<int64_t>(qin ? qrow : a.rows - 1) * a.ldq + hl * kHalf;
+#pragma unroll
+      for (int i = 0; i < kHalf; i += 4) {
+        const float4 t = *reinterpret_cast<const float4*>(p + i);
+        qv[i] = t.x;
+        qv[i + 1] = t.y;
+        qv[i + 2] = t.z;
+        qv[i + 3] = t.w;
+      }
+    }
+    // the n-th live tile past u of the words (kWalkTiles: none)
+    auto advance = [&](int u, int n) {
+      for (;;) {
+        ++u;
+        if (u >= kWalkTiles) return kWalkTiles;
+        const uint32_t w = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(word), u >> 5)) >> (u & 31);
+        if (w == 0) {
+          u |= 31;
+        } else {
+          u += __builtin_ctz(w);
+          if (--n == 0) return u;
+        }
+      }
+    };
+    int t = advance(-1, wave + 1);
+    if (t < kWalkTiles) {
+      stage_k(base + t);
+      stage_v(base + t);
+    }
+    while (t < kWalkTiles) {
+      const int next = advance(t, kWalkWaves);
+      wait_loads<kTileLoads, false>();  // K and the mask are in LDS, V may be on its way
+      __builtin_amdgcn_sched_barrier(0);
+      // the lane's byte offsets in the tiles, formed anew for each tile: kept,
+      // the 16 of K alone are registers the accumulators need
+      uint32_t k_at = 4 * HD * c + 16 * ((hl * (kHalf / 4)) ^ (c & 15));
+      uint32_t m_at = 4 * kKeyTile * c + 16 * (hl ^ ((c >> 1) & 7));
+      uint32_t v_at = 4 * (4 * hl * HD + (c ^ (32 * hl)));
+      asm volatile("" : "+v"(k_at), "+v"(m_at), "+v"(v_at));
+      float mk[16];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const float4 x = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(ms) + (m_at ^ (32 * g)));
+        mk[4 * g] = x.x;
+        mk[4 * g + 1] = x.y;
+        mk[4 * g + 2] = x.z;
+        mk[4 * g + 3] = x.w;
+      }
+      // S^T = K Q^T: 32 keys x 32 queries
+      f32x16 s;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = 0.0f;
+#pragma unroll
+      for (int i = 0; i < kHalf; i += 4) {
+        const float4 kk = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(ks) + (k_at ^ (4 * i)));
+        s = __builtin_amdgcn_mfma_f32_32x32x2f32(kk.x, qv[i], s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_32x32x2f32(kk.y, qv[i + 1], s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_32x32x2f32(kk.z, qv[i + 2], s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_32x32x2f32(kk.w, qv[i + 3], s, 0, 0, 0);
+      }
+      // one wave a SIMD: the LDS reads go out four products' groups ahead, or
+      // every group would wait for its own
+      constexpr int kMfma = 0x008, kDsRead = 0x100, kAhead = 4;
+      __builtin_amdgcn_sched_group_barrier(kDsRead, 4 + kAhead, 0);  // the mask's and the first of K's
+#pragma unroll
+      for (int i = 0; i < kHalf / 4 - kAhead; ++i) {
+        __builtin_amdgcn_sched_group_barrier(kMfma, 4, 0);
+        __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(kMfma, 4 * kAhead, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      float tmax = -INFINITY;
+      const int left = a.keys - (base + t) * kKeyTile - 4 * hl;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float x = s[r] * a.scale + mk[r];
+        s[r] = 8 * (r / 4) + r % 4 < left ? x : -INFINITY;
+        tmax = fmaxf(tmax, s[r]);
+      }
+      if (next < kWalkTiles) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this tile's K and mask are read
+        stage_k(base + next);
+      }
+      tmax = fmaxf(tmax, partner(tmax));
+      const float m_new = fmaxf(m, tmax);
+      const bool dead = m_new == -INFINITY;  // nothing finite yet
+      const float corr = dead ? 1.0f : __builtin_amdgcn_exp2f((m - m_new) * kLog2e);
+      float psum = 0.0f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        s[r] = dead ? 0.0f : __builtin_amdgcn_exp2f((s[r] - m_new) * kLog2e);
+        psum += s[r];
+      }
+      psum += partner(psum);
+      l = l * corr + psum;
+      m = m_new;
+      if (__ballot(corr != 1.0f) != 0) {
+#pragma unroll
+        for (int b = 0; b < kDBlocks; ++b) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[b][r] *= corr;
+        }
+      }
+      // V is in LDS; the next K and mask may be on their way
+      if (next < kWalkTiles) {
+        wait_loads<kTileLoads + kMaskLoads, false>();
+      } else {
+        wait_loads<0, false>();
+      }
+      const int vkeys = a.keys - (base + t) * kKeyTile;
+      if (vkeys < kKeyTile) {  // uniform: zeros past the keys, whatever the last one holds
+        for (int i = lane; i < (kKeyTile - vkeys) * HD; i += kWave) vs[vkeys * HD + i] = 0.0f;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      }
+      // O^T += V^T P^T: product r sums keys 8 (r / 4) + 4 h + r % 4, held in s[r]
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const char* vrow = reinterpret_cast<const char*>(vs) + 4 * (8 * (r / 4) + r % 4) * HD;
+#pragma unroll
+        for (int b = 0; b < kDBlocks; ++b) {
+          const uint32_t at = (b & 1) != 0 ? v_at ^ 128u : v_at;
+          const float x = *reinterpret_cast<const float*>(vrow + at + 256 * (b / 2));
+          o[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, s[r], o[b], 0, 0, 0);
+        }
+      }
+      __builtin_amdgcn_sched_group_barrier(kDsRead, 2 * kDBlocks, 0);  // (of one dword: two rows ahead)
+#pragma unroll
+      for (int i = 0; i < 14; ++i) {
+        __builtin_amdgcn_sched_group_barrier(kMfma, kDBlocks, 0);
+        __builtin_amdgcn_sched_group_barrier(kDsRead, kDBlocks, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(kMfma, 2 * kDBlocks, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (next < kWalkTiles) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this tile's V is read
+        stage_v(base + next);
+      }
+      t = next;
+    }
+  }
+
+  // the four records of each row through LDS, in the tiles' place
+  float* const vals = stages;
+  float* const mx = stages + kVals;
+  float* const tot = mx + kWalkWaves * kQueriesPerWave;
+  __syncthreads();
+#pragma unroll
+  for (int b = 0; b < kDBlocks; ++b) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      *reinterpret_cast<float4*>(vals + (wave * kQueriesPerWave + c) * kP + 32 * b + 8 * g + 4 * hl) =
+          make_float4(o[b][4 * g], o[b][4 * g + 1], o[b][4 * g + 2], o[b][4 * g + 3]);
+    }
+  }
+  if (hl == 0) {
+    mx[wave * kQueriesPerWave + c] = m;
+    tot[wave * kQueriesPerWave + c] = l;
+  }
+  __syncthreads();
+  // thread: row threadIdx.x / 8, columns 4 (threadIdx.x % 8) + 32 b .. + 3
+  const int row = static_cast<int>(threadIdx.x) / 8, d0 = 4 * (static_cast<int>(threadIdx.x) % 8);
+  if (q0 + row >= a.rows) return;
+  float big = -INFINITY;
+#pragma unroll
+  for (int w = 0; w < kWalkWaves; ++w) big = fmaxf(big, mx[w * kQueriesPerWave + row]);
+  float e[kWalkWaves], total = 0.0f;
+#pragma unroll
+  for (int w = 0; w < kWalkWaves; ++w) {
+    const float mw = mx[w * kQueriesPerWave + row];
+    e[w] = mw == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((mw - big) * kLog2e);
+    total += e[w] * tot[w * kQueriesPerWave + row];
+  }
+  const bool record = block_runs > 1;  // the run's (m, l) and O unnormalised
+  const float inv = record ? 1.0f : total > 0.0f ? 1.0f / total : 0.0f;
+  const int64_t rec = ((slice * ((a.rows + 4 * kQueriesPerWave - 1) / (4 * kQueriesPerWave)) + rblk) * a.runs + run) *
+                          (4 * kQueriesPerWave) +
+                      (q0 + row - rblk * 4 * kQueriesPerWave);
+  if (record && d0 == 0) *reinterpret_cast<float2*>(a.part_ml + 2 * rec) = make_float2(big, total);
+  const int64_t orow = slice_at(a, slice, a.so, a.io) + static_cast<int64_t>(q0 + row) * a.ldo;
+#pragma unroll
+  for (int b = 0; b < kDBlocks; ++b) {
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int w = 0; w < kWalkWaves; ++w) {
+      const float4 x = *reinterpret_cast<const float4*>(vals + (w * kQueriesPerWave + row) * kP + 32 * b + d0);
+      acc[0] += e[w] * x.x;
+      acc[1] += e[w] * x.y;
+      acc[2] += e[w] * x.z;
+      acc[3] += e[w] * x.w;
+    }
+    if (record) {
+      *reinterpret_cast<float4*>(a.part_o + rec * HD + 32 * b + d0) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+    } else {
+      store4(a, orow + 32 * b + d0, acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
+    }
+  }
+}
+
 // The relative-position dot products of every (slice, query row) into
 // table [slices][rows][dots_ld] (height terms at 0, width terms at dw_off),
 // on the fp32 matrix cores: block (j, s) takes table slice j of slice s
@@ -1747,6 +2059,43 @@ int launch(const char* what, void* stream, int64_t hd, int64_t slices, const Att
   } else {
     allow_lds(attention_k<128, kBias>, dyn);
     attention_k<128, kBias><<<grid, kThreads, dyn, as_stream(stream)>>>(a);
+  }
+  return check_launch(what);
+}
+
+// attention with a mask, over a's map and runs where it has them.
+int launch_mask(const char* what, void* stream, int64_t hd, int64_t slices, const AttnArgs& a) {
+  constexpr int64_t kMost = int64_t{1} << 23;  // workgroups a launch (of 256 threads, below 2^32 in all)
+  const int64_t groups = (a.rows + int64_t{kQueriesPerWave} - 1) / kQueriesPerWave;
+  const int64_t part = groups * a.runs <= kMost ? groups : kMost / a.runs;  // row groups and slices a launch
+  const int64_t per = kMost / (part * a.runs);
+  clear_launch_error();
+  for (int64_t s = 0; s < slices; s += per) {
+    AttnArgs b = a;
+    b.q += s * a.sq;
+    b.k += s * a.sk;
+    b.v += s * a.sv;
+    if (a.out16 != nullptr) {
+      b.out16 += s * a.so;
+    } else {
+      b.out += s * a.so;
+    }
+    const int64_t records = s * ((a.rows + 127) / 128) * a.runs * 128;
+    if (a.part_o != nullptr) {
+      b.part_o += records * hd;
+      b.part_ml += 2 * records;
+    }
+    for (int64_t g = 0; g < groups; g += part) {
+      const int64_t here = groups - g < part ? groups - g : part;
+      const unsigned grid = static_cast<unsigned>((slices - s < per ? slices - s : per) * here * a.runs);
+      if (hd == 64) {
+        attention_mask_k<64><<<grid, 64 * kWalkWaves, 0, as_stream(stream)>>>(b, static_cast<int>(g),
+                                                                              static_cast<int>(here));
+      } else {
+        attention_mask_k<128><<<grid, 64 * kWalkWaves, 0, as_stream(stream)>>>(b, static_cast<int>(g),
+                                                                               static_cast<int>(here));
+      }
+    }
   }
   return check_launch(what);
 }
@@ -1902,8 +2251,7 @@ int attention_entry(const char* what, void* stream, const float* q, int64_t ldq,
     attention_keysplit_k<<<grid, 64 * kSplitWaves, kSplitLds, as_stream(stream)>>>(a);
     return check_launch(what);
   }
-  return mask != nullptr ? launch<Bias::kMask>(what, stream, hd, slices, a)
-                         : launch<Bias::kNone>(what, stream, hd, slices, a);
+  return mask != nullptr ? launch_mask(what, stream, hd, slices, a) : launch<Bias::kNone>(what, stream, hd, slices, a);
 }
 
 // The masked split-operand attention's workspace: the mask's tile map
@@ -1955,6 +2303,8 @@ int64_t fp32_workspace_floats(int64_t slices, int64_t rows, int64_t keys, int64_
   return masked_tiles_offset(rows, keys) + fp32_partial_rows(slices, rows, keys, hd) * (hd + 2);
 }
 
+constexpr int64_t kFewGroups = 128, kMapGroups = 1024;
+
 int masked_fp32_entry(const char* what, void* stream, const float* q, int64_t ldq, int64_t sq, const float* k,
                       int64_t ldk, int64_t sk, const float* v, int64_t ldv, int64_t sv, float* out, int64_t ldo,
                       int64_t so, int64_t slices, int64_t rows, int64_t keys, int64_t hd, float scale,
@@ -1976,7 +2326,14 @@ int masked_fp32_entry(const char* what, void* stream, const float* q, int64_t ld
   AttnArgs a{q, k, v, out, ldq, sq, ldk, sk, ldv, sv, ldo, so, static_cast<int>(rows), static_cast<int>(keys),
              scale, mask, mask_ld, nullptr, nullptr, 0, 0, 0, 0, nullptr, nullptr, 1, 0, 0, 0, 0, out16};
   if (out16 != nullptr) a.out = nullptr;
-  const int64_t runs = masked_runs(slices, rows, keys, fp32_slots(hd));
+  // The map (15 us at 4096 x 4096) spares the scans of dead spans where there
+  // are row groups enough to keep every CU scanning (10 x 4096 x 128 routed 384
+  // us with it, 404 without; causal 687 / 714; at 12 x 300 x 64 over 1000
+  // keys 47 / 40), and the runs it cuts pay where the row groups leave CUs
+  // idle; between the two the mask alone is the faster.
+  const int64_t groups = slices * ((rows + kQueriesPerWave - 1) / kQueriesPerWave);
+  const int64_t runs = groups < kFewGroups ? masked_runs(slices, rows, keys, fp32_slots(hd)) : 1;
+  if (groups < kMapGroups && runs == 1) return launch_mask(what, stream, hd, slices, a);
   uint32_t* map = reinterpret_cast<uint32_t*>(workspace);
   a.map = map;
   a.map_words = static_cast<int>(words);
@@ -1991,15 +2348,8 @@ int masked_fp32_entry(const char* what, void* stream, const float* q, int64_t ld
                  as_stream(stream)>>>(
       mask, mask_ld, static_cast<int>(rows), static_cast<int>(keys), map, static_cast<int>(words));
   if (const int st = check_launch(what)) return st;
-  const dim3 grid(static_cast<unsigned>(row_blocks * runs), static_cast<unsigned>(slices));
-  clear_launch_error();
-  if (hd == 64) {
-    attention_k<64, Bias::kMask><<<grid, 256, 0, as_stream(stream)>>>(a);
-  } else {
-    attention_k<128, Bias::kMask><<<grid, 256, 0, as_stream(stream)>>>(a);
-  }
-  if (runs == 1) return check_launch(what);
-  if (const int st = check_launch(what)) return st;
+  if (const int st = launch_mask(what, stream, hd, slices, a)) return st;
+  if (runs == 1) return UOCR_ROCM_OK;
   X3Partials part{a.run_tiles, a.runs, a.part_o, a.part_ml};
   const dim3 merge_grid(static_cast<unsigned>(row_blocks), static_cast<unsigned>(slices));
   clear_launch_error();

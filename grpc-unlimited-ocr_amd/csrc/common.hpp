@@ -249,6 +249,42 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// ---- memory to LDS ------------------------------------------------------------
+
+typedef __attribute__((address_space(3))) void* LdsPtr;
+
+// The LDS address of a wave-uniform pointer into a __shared__ array.
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+  return __builtin_amdgcn_readfirstlane(
+      static_cast<uint32_t>(reinterpret_cast<uintptr_t>((LdsPtr) const_cast<void*>(p))));
+}
+
+// One 16-byte memory-to-LDS load a lane: lane l's bytes go to LDS address
+// lds + 16 l. In assembly because the compiler puts a wait for every
+// outstanding load of the builtin's form before the next LDS read, which
+// takes the next step's loads into this step's time (a 64 x 64 tile's step of
+// 64 columns then lasts a whole memory latency, 0.85 us); the callers wait
+// with counts of their own before they read.
+__device__ __forceinline__ void dma16(uint32_t lds, const char* base, uint32_t off) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
+               : "memory");
+}
+__device__ __forceinline__ void dma16(uint32_t lds, const char* base, uint64_t off) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(base + off)
+               : "memory");
+}
+
+// At most kPending of this wave's memory loads outstanding and all its LDS
+// reads returned; with kBarrier, then the workgroup's barrier.
+template <int kPending, bool kBarrier>
+__device__ __forceinline__ void wait_loads() {
+  if constexpr (kBarrier) {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kPending) : "memory");
+  } else {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kPending) : "memory");
+  }
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
   v += dpp_f32<0xB1>(v);   // quad_perm [1,0,3,2]: partner lane ^ 1
   v += dpp_f32<0x4E>(v);   // quad_perm [2,3,0,1]: partner lane ^ 2

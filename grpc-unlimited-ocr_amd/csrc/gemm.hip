@@ -432,34 +432,6 @@ __global__ __launch_bounds__(kGemmThreads) void linear_staged_k(const LinearArgs
   }
 }
 
-typedef __attribute__((address_space(3))) void* LdsPtr;
-
-// One 16-byte memory-to-LDS load a lane: lane l's bytes go to LDS address
-// lds + 16 l. In assembly because the compiler puts a wait for every
-// outstanding load of the builtin's form before the next LDS read, which
-// takes the next step's loads into this step's time (a 64 x 64 tile's step of
-// 64 columns then lasts a whole memory latency, 0.85 us); the callers wait
-// with counts of their own before they read.
-__device__ __forceinline__ void dma16(uint32_t lds, const char* base, uint32_t off) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
-               : "memory");
-}
-__device__ __forceinline__ void dma16(uint32_t lds, const char* base, uint64_t off) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(base + off)
-               : "memory");
-}
-
-// At most kPending of this wave's memory loads outstanding and all its LDS
-// reads returned; with kBarrier, then the workgroup's barrier.
-template <int kPending, bool kBarrier>
-__device__ __forceinline__ void wait_loads() {
-  if constexpr (kBarrier) {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kPending) : "memory");
-  } else {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kPending) : "memory");
-  }
-}
-
 // A tile of TM x TN outputs by WM x WN x WK waves; kKC columns of k a step,
 // kS steps of tiles in LDS, kS - 1 of them in flight ahead of the products.
 //
@@ -521,8 +493,7 @@ __global__ __launch_bounds__(kWave* WM* WN* WK) void linear_pipe_k(const LinearA
     off[i] = static_cast<Off>(row < last ? row : last) * a.k * 2 + c * 16;
   }
   u32x4* const mine = lds + grp * kS * kStage;
-  const uint32_t lds0 =
-      __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((LdsPtr)mine)));
+  const uint32_t lds0 = lds_address(mine);
   auto issue = [&](int t, int buf) {
     const int64_t at = static_cast<int64_t>(t) * kKC * 2;
 #pragma unroll

@@ -378,3 +378,75 @@ def test_attention_masked_refuses_what_it_cannot_take(backend):
         backend.attention_masked(q, q, q, out, 1, 64, 64, 128, 0.1, m2, ws)
     with pytest.raises(ValueError):  # an fp32 out
         backend.attention_masked(q, q, q, q, 1, 64, 64, 128, 0.1, mask, ws)
+
+
+@pytest.mark.parametrize("slices,rows,keys,hd,kind,ld", [
+    (40, 830, 96, 64, "random", 96), (36, 930, 71, 128, "random", 72),  # row groups enough for the map
+    (2, 33, 33000, 64, "sparse", 33000), (1, 5, 33003, 128, "sparse", 33003),  # past the tiles of one scan
+    (3, 70, 255, 128, "random", 257), (2, 31, 64, 64, "random", 65),  # mask rows off 16 bytes
+    (5, 257, 1, 64, "causal", 4), (1, 64, 4100, 128, "dead", 4100)])
+@pytest.mark.parametrize("workspace", [False, True])
+def test_attention_mask_walk(backend, slices, rows, keys, hd, kind, ld, workspace):
+    """The masked attention's walk at its edges: partial tiles and row groups,
+    scans of more than 1024 tiles, mask rows that allow no 16-byte reads, with
+    the map of a workspace, with runs and without either, at the fp32 bar."""
+    g = np.random.default_rng(slices + rows + keys)
+    q, k, v = (normal(800 + i, (slices, n, hd)) for i, n in enumerate((rows, keys, keys)))
+    mask = (0.1 * g.standard_normal((rows, keys))).astype(np.float32)
+    if kind == "causal":
+        mask[np.arange(keys)[None] > np.arange(rows)[:, None]] = -np.inf
+    elif kind == "sparse":
+        mask[:] = -np.inf
+        for r in range(rows):
+            mask[r, g.integers(0, keys, 40)] = 0.5
+        mask[:, keys - 1] = 0.0
+    else:
+        mask[g.random((rows, keys)) < 0.7] = -np.inf
+    if kind == "dead":
+        mask[:32] = -np.inf
+        mask[40:, 64:4064] = -np.inf
+    wide = np.full((rows, ld), np.nan, np.float32)  # columns past the keys are not read
+    wide[:, :keys] = mask
+    out = torch.full((slices, rows, hd), float("nan"), device="cuda")
+    ws = torch.full((backend.attention_workspace_floats(slices, rows, keys, hd),), float("nan"), device="cuda")
+    backend.attention(dev_f32(q), dev_f32(k), dev_f32(v), out, slices, rows, keys, hd, 0.1, mask=dev_f32(wide),
+                      workspace=ws if workspace else None)
+    got = host_f32(out)
+    dead = ~np.isfinite(mask).any(axis=1)
+    assert np.array_equal(got[:, dead], np.zeros_like(got[:, dead]))
+    assert_f32_close(got, reference(q, k, v, 0.1, mask), 1e-5, f"mask walk {kind}")
+
+
+def test_attention_mask_far_rows(backend):
+    """Key and value rows 2^24 floats apart (past the walk's 32-bit lane
+    offsets): the packed rows' output, bitwise."""
+    rows, keys, hd, ld = 3, 5, 64, 1 << 24
+    q, k, v = normal(820, (rows, hd)), normal(821, (keys, hd)), normal(822, (keys, hd))
+    mask = np.zeros((rows, keys), np.float32)
+    mask[1, 2] = -np.inf
+    want, got = (torch.full((1, rows, hd), float("nan"), device="cuda") for _ in range(2))
+    backend.attention(dev_f32(q), dev_f32(k), dev_f32(v), want, 1, rows, keys, hd, 0.1, mask=dev_f32(mask))
+    far = torch.empty((keys - 1) * ld + 2 * hd, device="cuda")
+    for i in range(keys):
+        far[i * ld:i * ld + hd] = dev_f32(k)[i]
+        far[i * ld + hd:i * ld + 2 * hd] = dev_f32(v)[i]
+    backend.attention(dev_f32(q), far, far, got, 1, rows, keys, hd, 0.1, mask=dev_f32(mask),
+                      strides={"k": (0, ld, 0), "v": (hd, ld, 0)})
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("keys", [96, 90])
+def test_attention_mask_infinite_values(backend, keys):
+    """An infinite value row in a tile that only the second row group reads:
+    the first group's rows are untouched by it; keys past the end bring no
+    copy of the last value row into a product."""
+    rows, hd = 64, 64
+    q, k, v = normal(830, (rows, hd)), normal(831, (keys, hd)), normal(832, (keys, hd))
+    v[keys - 1] = np.inf
+    mask = np.zeros((rows, keys), np.float32)
+    mask[:32, 64:] = -np.inf
+    out = torch.full((1, rows, hd), float("nan"), device="cuda")
+    backend.attention(dev_f32(q), dev_f32(k), dev_f32(v), out, 1, rows, keys, hd, 0.1, mask=dev_f32(mask))
+    got = host_f32(out)[0]
+    assert_f32_close(got[:32], reference(q[None], k[None], np.where(np.isinf(v), 0, v)[None], 0.1, mask)[0, :32], 1e-5, "rows before")
+    assert np.all(got[32:] == np.inf)
