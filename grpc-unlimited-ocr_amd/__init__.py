@@ -680,8 +680,8 @@ def attention(q, k, v, out, slices, rows, keys, hd, scale, mask=None, strides=No
     """out[s, t] = softmax(scale q[s, t] . k[s, :] + mask[t, :]) v[s, :] in one
     pass (new). strides: {name: (offset, ld, slice_stride)} for q, k, v, out
     (elements); default head-major [slices, rows or keys, hd]. workspace
-    (attention_workspace_floats floats): a mask's live tiles walked alone,
-    long walks cut into runs merged by a last launch."""
+    (attention_workspace_floats floats): a map of a mask's live tiles for many
+    query rows, for few the walks cut into runs merged by a last launch."""
     st = strides or {}
     qo = _operand(q, *st.get("q", (0, hd, rows * hd)))
     ko = _operand(k, *st.get("k", (0, hd, keys * hd)))

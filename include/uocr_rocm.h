@@ -519,11 +519,12 @@ UOCR_ROCM_API int uocr_rocm_attention_bf16(void* stream, const float* q, int64_t
                                            int64_t mask_ld);
 /* New: uocr_rocm_attention and uocr_rocm_attention_bf16 with a workspace
  * (uocr_rocm_attention_workspace_floats(slices, rows, keys, hd) floats,
- * 16-byte aligned) for a mask: a first launch marks, per 128 query rows,
- * the 32-key tiles where some mask entry is finite, and the fp32 products
- * walk only those; where the row blocks of all slices leave CUs idle, a
- * block's walk is cut into runs whose (max, total, values) records a last
- * launch combines, so a causal mask's longest walks no longer set the time.
+ * 16-byte aligned) for a mask: with many query rows a first launch marks,
+ * per 128 of them, the 32-key tiles where some mask entry is finite, and only
+ * those are looked at for a row group's live tiles; with few, whose row blocks
+ * leave CUs idle, a block's walk is cut by that map into runs whose (max,
+ * total, values) records a last launch combines; between the two the
+ * workspace is unused.
  * fp32 arithmetic throughout (the sums of a cut row in another order); the
  * bf16 entry is bitwise the fp32 one then uocr_rocm_round_bf16. A null mask
  * takes the entries above (the workspace unused). */
