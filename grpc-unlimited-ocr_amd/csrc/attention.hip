@@ -1530,20 +1530,23 @@ __global__ __launch_bounds__(64 * kSplitWaves) void attention_keysplit_k(const A
 // into runs, whose records x3m_merge_k combines.
 //
 // us, 128 rows a workgroup before / now (10 heads x 4096 x 128): routed 720 /
-// 384, causal 1231 / 687; 12 x 300 x 64 over 1000 keys causal 122 / 45. A live
-// tile takes a wave 13000 clocks at head dim 128, the matrix cores 8192 of
-// them; one workgroup holds a CU's LDS, so its scan (5 TB/s of mask over the
-// chip) and its first reads stand alone. Half the LDS and two workgroups a CU
-// (K and V in turn in one place) had the accumulators spill and took 498 us
-// routed; K and V read by the lanes that use them, without LDS, 421.
+// 374, causal 1231 / 656; head dim 64: 12 x 300 over 1000 keys causal 122 / 44,
+// 12 x 4096 causal 663 / 444. A live tile takes a wave 12700 clocks at head
+// dim 128, the matrix cores 8192 of them; one workgroup holds a CU's LDS, so
+// its scan (5 TB/s of mask over the chip) and its first reads stand alone. At
+// head dim 64 two fit a CU (12 x 4096 551 to 444 us), for which the scan keeps
+// 8 rows in flight, not 16, or its registers would not leave room. At 128
+// half the LDS and two workgroups (K and V in turn in one place) had the
+// accumulators spill and took 498 us routed; K and V read by the lanes that
+// use them, without LDS, 421.
 constexpr int kWalkTiles = 1024;  // tiles a scan covers
 constexpr int kWalkWaves = 4;
-constexpr int kScanRows = 16;
 
 template <int HD>
-__global__ __launch_bounds__(64 * kWalkWaves, 1) void attention_mask_k(const AttnArgs a, int first_group,
+__global__ __launch_bounds__(64 * kWalkWaves, HD == 64 ? 2 : 1) void attention_mask_k(const AttnArgs a, int first_group,
                                                                      int row_groups) {
   constexpr int kHalf = HD / 2, kDBlocks = HD / 32, kP = HD + 4;
+  constexpr int kScanRows = HD == 64 ? 8 : 16;
   constexpr int kTileElems = kKeyTile * HD, kMaskElems = kQueriesPerWave * kKeyTile;
   constexpr int kStage = 2 * kTileElems + kMaskElems;  // a wave's K, V and mask tiles
   // 144 KB at head dim 128. The live words take the tiles' place before a walk,
@@ -1676,7 +1679,7 @@ __global__ __launch_bounds__(64 * kWalkWaves, 1) void attention_mask_k(const Att
         // read the last ones), so that kScanRows rows are in flight at once
         const int key4 = t8 * kKeyTile + 4 * lane;
         const int rlast = a.rows - 1 - q0 < kQueriesPerWave ? a.rows - 1 - q0 : kQueriesPerWave - 1;
-        const float* const mp = a.mask + static_cast<int64_t>(q0) * a.mask_ld;
+        const float* row = a.mask + static_cast<int64_t>(q0) * a.mask_ld;
         bool any = false;
 #pragma unroll
         for (int half = 0; half < kQueriesPerWave; half += kScanRows) {
@@ -1685,15 +1688,16 @@ __global__ __launch_bounds__(64 * kWalkWaves, 1) void attention_mask_k(const Att
             const int at4 = key4 < a.keys ? key4 : (a.keys - 1) & ~3;
 #pragma unroll
             for (int r = 0; r < kScanRows; ++r) {
-              x[r] = *reinterpret_cast<const float4*>(mp + static_cast<int64_t>(min(half + r, rlast)) * ld + at4);
+              x[r] = *reinterpret_cast<const float4*>(row + at4);
+              row += half + r < rlast ? ld : 0;
             }
           } else {
             const int k0 = min(key4, a.keys - 1), k1 = min(key4 + 1, a.keys - 1), k2 = min(key4 + 2, a.keys - 1),
                       k3 = min(key4 + 3, a.keys - 1);
 #pragma unroll
             for (int r = 0; r < kScanRows; ++r) {
-              const float* const row = mp + static_cast<int64_t>(min(half + r, rlast)) * ld;
               x[r] = make_float4(row[k0], row[k1], row[k2], row[k3]);
+              row += half + r < rlast ? ld : 0;
             }
           }
 #pragma unroll
@@ -2327,9 +2331,9 @@ int masked_fp32_entry(const char* what, void* stream, const float* q, int64_t ld
              scale, mask, mask_ld, nullptr, nullptr, 0, 0, 0, 0, nullptr, nullptr, 1, 0, 0, 0, 0, out16};
   if (out16 != nullptr) a.out = nullptr;
   // The map (15 us at 4096 x 4096) spares the scans of dead spans where there
-  // are row groups enough to keep every CU scanning (10 x 4096 x 128 routed 384
-  // us with it, 404 without; causal 687 / 714; at 12 x 300 x 64 over 1000
-  // keys 47 / 40), and the runs it cuts pay where the row groups leave CUs
+  // are row groups enough to keep every CU scanning (10 x 4096 x 128 routed 374
+  // us with it, 395 without; causal 656 / 688; with it and no runs at 12 x 300
+  // x 64 over 1000 keys 47 / 40), and the runs it cuts pay where the row groups leave CUs
   // idle; between the two the mask alone is the faster.
   const int64_t groups = slices * ((rows + kQueriesPerWave - 1) / kQueriesPerWave);
   const int64_t runs = groups < kFewGroups ? masked_runs(slices, rows, keys, fp32_slots(hd)) : 1;
