@@ -264,7 +264,8 @@ __device__ __forceinline__ uint32_t lds_address(const void* p) {
 // outstanding load of the builtin's form before the next LDS read, which
 // takes the next step's loads into this step's time (a 64 x 64 tile's step of
 // 64 columns then lasts a whole memory latency, 0.85 us); the callers wait
-// with counts of their own before they read.
+// with counts of their own before they read. (m0 is a reserved register: no
+// other instruction of these kernels sets or reads it.)
 __device__ __forceinline__ void dma16(uint32_t lds, const char* base, uint32_t off) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
                : "memory");
